@@ -432,14 +432,13 @@ __global__ void __launch_bounds__(256) k_nn_head_bwd(long tot, const uint16_t* _
 
 // One layer backward.  In: h^{l} (Hin), dh^{l+1} (dH).  Out: dHp = dH + W_h^T dz,
 // dM = W_m^T dz (aggregated into dh^{l} by k_nn_agg_bwd), per-wave partials of
-// dW (32x64) and db (32).  Every wave of a workgroup runs the same number of
+// dW (32x64) and db (32) into `part`.  Every wave of a workgroup runs the same number of
 // iterations (tiles past the end are masked) so the LDS barriers line up.
 __global__ void __launch_bounds__(256) k_nn_layer_bwd(Graph G, const uint16_t* __restrict__ Hin,
                                                       const float* __restrict__ dH, const uint16_t* __restrict__ W,
                                                       const uint16_t* __restrict__ WT, const float* __restrict__ b,
                                                       float* __restrict__ dHp, float* __restrict__ dM,
-                                                      float* __restrict__ dWpart, float* __restrict__ dbpart,
-                                                      long ntiles) {
+                                                      float* __restrict__ part, long ntiles) {
   __shared__ uint16_t lds_dzT[4][32 * 32];   // [cell][channel]
   __shared__ uint16_t lds_dzN[4][32 * 32];   // [channel][cell]
   __shared__ uint16_t lds_hmN[4][64 * 32];   // [channel][cell]
@@ -535,9 +534,9 @@ __global__ void __launch_bounds__(256) k_nn_layer_bwd(Graph G, const uint16_t* _
     }
     __syncthreads();
   }
-  // per-wave partials: dW[out][in] (out = accumulator row, in = column)
-  const long gw = (long)blockIdx.x * 4 + wv;
-  float* dw = dWpart + gw * (kC * 2 * kC);
+  // per-wave partials, laid out as a layer's parameters: dW[out][in] (out =
+  // accumulator row, in = column), then db[out]
+  float* dw = part + ((long)blockIdx.x * 4 + wv) * kLayer;
 #pragma unroll
   for (int r = 0; r < 16; ++r) {
     const int out = acc_row(r, half);
@@ -554,7 +553,7 @@ __global__ void __launch_bounds__(256) k_nn_layer_bwd(Graph G, const uint16_t* _
   }
   if (col == 0) {
 #pragma unroll
-    for (int r = 0; r < 16; ++r) dbpart[gw * kC + acc_row(r, half)] = dbacc[r];
+    for (int r = 0; r < 16; ++r) dw[kC * 2 * kC + acc_row(r, half)] = dbacc[r];
   }
 }
 
@@ -587,23 +586,38 @@ __global__ void __launch_bounds__(256) k_nn_agg_bwd(Graph G, const float* __rest
   }
 }
 
-// out[k] = sum_p part[p*len + k] (fixed order, double accumulation)
-__global__ void k_nn_reduce(const float* __restrict__ part, long nparts, int len, float* __restrict__ out) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= len) return;
+// out[k] = sum_p part[p*len + k] for k < split, out[k + gap] for the rest (double
+// accumulation).  A workgroup owns kRedCols columns: thread (r, c) adds rows
+// r, r + kRedRows, ... of column c, eight loads in flight, and the kRedRows
+// sums are added in order.  Bound by reading the partials (a row segment is
+// 64 bytes): 4096 partials of 2080 floats go through 130 workgroups, where
+// one thread per column (nine workgroups) was a serial chain of 4096 loads.
+// At 4 systems of 512^2, a layer: 1210 us before, 12.5 us now (2.7 TB/s).
+constexpr int kRedCols = 16, kRedRows = 1024 / kRedCols;
+__global__ void __launch_bounds__(1024) k_nn_reduce(const float* __restrict__ part, long nparts, int len,
+                                                    float* __restrict__ out, int split, int gap) {
+  __shared__ double sh[kRedRows][kRedCols + 1];
+  const int c = threadIdx.x % kRedCols, r = threadIdx.x / kRedCols;
+  const int k = blockIdx.x * kRedCols + c;
   double acc = 0.0;
-  for (long p = 0; p < nparts; ++p) acc += (double)part[p * len + k];
-  out[k] = (float)acc;
-}
-
-// head partial layout (5*32 pairs then 5 biases) -> grad
-__global__ void k_nn_reduce_head(const float* __restrict__ part, long nparts, float* __restrict__ grad) {
-  const int t = threadIdx.x;
-  if (t >= 5 * kC + 5) return;
-  double acc = 0.0;
-  for (long p = 0; p < nparts; ++p) acc += (double)part[p * (5 * kC + 5) + t];
-  if (t < 5 * kC) grad[kOffWo + t] = (float)acc;  // rows 0..4 of Wo (row-major [k][c])
-  else grad[kOffBo + (t - 5 * kC)] = (float)acc;
+  if (k < len) {
+    long p = r;
+    for (; p + 7L * kRedRows < nparts; p += 8L * kRedRows) {
+      float v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = part[(p + (long)u * kRedRows) * len + k];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) acc += (double)v[u];
+    }
+    for (; p < nparts; p += kRedRows) acc += (double)part[p * len + k];
+  }
+  sh[r][c] = acc;
+  __syncthreads();
+  if (r == 0 && k < len) {
+    double t = 0.0;
+    for (int q = 0; q < kRedRows; ++q) t += sh[q][c];
+    out[k < split ? k : k + gap] = (float)t;
+  }
 }
 
 // BF16 copies of the layer weights, row-major W[l][out][in] and W^T[l][in][out]
@@ -708,7 +722,7 @@ struct Trainer {
   DevBuf<float> pool_sd, pool_xh, pool_bh;
   std::vector<double> bnorm2;  // ||bh||^2 per pooled system
   Work w;
-  DevBuf<float> xh, bh, Lh, u, r, wv, dO, dH, dHp, dM, grad, m, v, part_w, part_b, part_h;
+  DevBuf<float> xh, bh, Lh, u, r, wv, dO, dH, dHp, dM, grad, m, v, part_l, part_h;
   DevBuf<double> rpart, gsc;
   long adam_t = 0;
   int nbs = 0;
@@ -835,24 +849,24 @@ double loss_grad(Trainer& T, const int* idx, int S) {
   PARCEL_HIP_CHECK(hipMemsetAsync(T.grad.p, 0, sizeof(float) * kNParam, st));
   hipLaunchKernelGGL(k_nn_head_bwd, dim3(hb), dim3(256), 0, st, tot, (const uint16_t*)T.w.H[kNL].p,
                      (const float*)T.dO.p, (const float*)N.P.p, T.dH.p, T.part_h.p);
-  hipLaunchKernelGGL(k_nn_reduce_head, dim3(1), dim3(256), 0, st, (const float*)T.part_h.p, (long)hb, T.grad.p);
+  // a partial holds rows 0..4 of dWo, then the 5 biases
+  hipLaunchKernelGGL(k_nn_reduce, dim3((5 * kC + 5 + kRedCols - 1) / kRedCols), dim3(1024), 0, st,
+                     (const float*)T.part_h.p, (long)hb, 5 * kC + 5, T.grad.p + kOffWo, 5 * kC,
+                     kOffBo - kOffWo - 5 * kC);
   // layers, last to first
   const Graph G{T.w.ahat.p, n, nx, S};
   const long ntiles = (long)S * (((long)n + 31) / 32);
   const unsigned lb = (unsigned)std::max<long>(1, std::min<long>((ntiles + 3) / 4, 1024));
   const long nw = (long)lb * 4;
-  if (T.part_w.n < (size_t)nw * kC * 2 * kC) T.part_w.alloc((size_t)nw * kC * 2 * kC);
-  if (T.part_b.n < (size_t)nw * kC) T.part_b.alloc((size_t)nw * kC);
+  if (T.part_l.n < (size_t)nw * kLayer) T.part_l.alloc((size_t)nw * kLayer);
   for (int l = kNL - 1; l >= 0; --l) {
     hipLaunchKernelGGL(k_nn_layer_bwd, dim3(lb), dim3(256), 0, st, G, (const uint16_t*)T.w.H[l].p,
                        (const float*)T.dH.p, (const uint16_t*)(N.W.p + (long)l * kC * 2 * kC),
                        (const uint16_t*)(N.WT.p + (long)l * kC * 2 * kC),
-                       (const float*)(N.P.p + (long)l * kLayer + kC * 2 * kC), T.dHp.p, T.dM.p, T.part_w.p,
-                       T.part_b.p, ntiles);
-    hipLaunchKernelGGL(k_nn_reduce, dim3((kC * 2 * kC + 255) / 256), dim3(256), 0, st, (const float*)T.part_w.p, nw,
-                       kC * 2 * kC, T.grad.p + (long)l * kLayer);
-    hipLaunchKernelGGL(k_nn_reduce, dim3(1), dim3(256), 0, st, (const float*)T.part_b.p, nw, kC,
-                       T.grad.p + (long)l * kLayer + kC * 2 * kC);
+                       (const float*)(N.P.p + (long)l * kLayer + kC * 2 * kC), T.dHp.p, T.dM.p, T.part_l.p,
+                       ntiles);
+    hipLaunchKernelGGL(k_nn_reduce, dim3((kLayer + kRedCols - 1) / kRedCols), dim3(1024), 0, st,
+                       (const float*)T.part_l.p, nw, kLayer, T.grad.p + (long)l * kLayer, kLayer, 0);
     if (l > 0)
       hipLaunchKernelGGL(k_nn_agg_bwd, dim3(grid_for(tot * (kC / 4))), dim3(256), 0, st, G, (const float*)T.dHp.p,
                          (const float*)T.dM.p, T.dH.p);

@@ -175,3 +175,11 @@ def test_mpnn_training_lowers_loss():
             its.append(int(niter.sum()))
     print("iterations untrained", its[0], "trained", its[1], flush=True)
     assert its[1] < its[0]
+
+
+@pytest.mark.parametrize("nx,ny", [(33, 31), (512, 40)])
+def test_mpnn_gradients_partial_counts(nx, ny):
+    # 256 and 1280 per-wavefront partials: the remainder loop of the sum over
+    # partials alone, and its unrolled rounds followed by a remainder; the
+    # bound is the BF16 one of the gradients
+    test_mpnn_gradients_match_oracle(nx, ny)
