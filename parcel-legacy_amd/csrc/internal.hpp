@@ -168,24 +168,37 @@ struct LscanBJ {
   DevBuf<double> sink;
 };
 
-// Line-wavefront form of the FP64 block-Jacobi apply: every block is whole
-// grid lines of nx cells (whole planes of ny lines, or lines of one plane)
-// whose factors couple a row only to the neighbouring cell of its line, the
-// same cell of the neighbouring line and of the neighbouring plane.  The
-// couplings (two per row, in the sweep's stored order) and the scales are
-// kept per block in anti-diagonal order of the sweep (precon.hip,
-// line_doff), so the rows one step of the wavefront visits are contiguous.
+// Line-wavefront form of the block-Jacobi apply: every block is a run of rows
+// of a natural-order grid whose factors couple a row only to the neighbouring
+// cell of its line, the same cell of the neighbouring line and of the
+// neighbouring plane (bjlines.hip).  Per sweep and wavefront the couplings
+// and scales lie in anti-diagonal order of the wavefront's lines, so the rows
+// of one step are contiguous.
+struct LineBlock {
+  int lo, len;   // the block's rows [lo, lo + len)
+  int ngf, ngb;  // groups of steps of the forward / backward sweep (even)
+};
+// One wavefront of a sweep: up to 64 consecutive lines of one plane.  Rows
+// are relative to the block's first row.
+struct LineWave {
+  int row0;   // first row (backward: last row) of lane 0's line, as if the line were whole
+  int nl;     // lines (0: an idle wavefront)
+  int tw;     // the step at which lane 0 computes cell 0
+  int hand;   // wavefront whose lane 63 holds the line before lane 0's (-1: none)
+  int plane;  // wavefront holding the same lines of the plane before (-1: none)
+  int pad;
+  long ebase; // first factor entry
+};
 struct LineBJ {
   bool on = false;
+  bool whole = false;     // every block is whole grid lines (and whole planes when it couples planes)
   int nx = 0;
-  int ny = 0;             // lines per plane when blocks hold several planes (0: one plane per block)
-  int planes = 1;         // most planes in a block
-  int waves = 1;          // wavefronts per workgroup: ceil(lines per plane / 64) x planes, rounded up to 2^k
-  DevBuf<int> bstart;     // nblocks + 1 block starts
-  DevBuf<double> fc, bc;  // line and cell couplings per row
-  DevBuf<double> fp, bp;  // plane coupling per row (several planes per block)
-  DevBuf<double> fd, bd;  // forward scale (D-ILU), backward scale
-  DevBuf<double> sink;    // 64 doubles per block for the stores of idle lanes
+  long nxy = 0;           // rows per plane (0: blocks do not couple planes)
+  int waves = 1;          // wavefronts per workgroup
+  DevBuf<LineBlock> blk;
+  DevBuf<LineWave> fw, bw;         // waves per block each
+  DevBuf<double> c[2][2];          // [forward, backward][hi, lo]: line and cell couplings per entry
+  DevBuf<double> e[2][2];          // plane coupling (blocks of several planes) and scale per entry
 };
 
 struct Precon {
@@ -197,7 +210,7 @@ struct Precon {
   DevBuf<float> dinv32;
   Sweep fwd, bwd;       // block Jacobi
   LscanBJ lscan;        // FP32 line-scan form of the block factors (mixed solver)
-  LineBJ line;          // line-wavefront form of the FP64 apply
+  LineBJ line;          // line-wavefront form of the FP64 or double-double apply
   bool has32 = false;   // FP32 copies of the factors exist
   // double-double factors (precon_setup_dd): Dinv lo parts, apply precision
   DevBuf<double> dinv_lo;

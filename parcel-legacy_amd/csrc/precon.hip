@@ -23,8 +23,8 @@
 #include <cstdlib>
 #include <cstring>
 
+#include "bj_sweep.hpp"
 #include "dd.hpp"
-#include "internal.hpp"
 
 namespace parcel {
 
@@ -67,19 +67,6 @@ void block_ranges(const Plan& P, int nblk, int n, std::vector<int>& blo, std::ve
   }
   for (int b = 0; b < nblk; ++b) divide_region0(b, nblk, n, &blo[b], &bhi[b]);
 }
-
-struct BlockSweep {
-  // rows of the block in level order, with per-level boundaries
-  std::vector<int> lev_start;   // offsets into order (size nlev+1)
-  std::vector<int> order;       // local rows (0-based within the block)
-  std::vector<int> ptr;         // entry ranges per local row (size nrow+1)
-  std::vector<int> dep;         // local dependency rows
-  std::vector<double> val;
-  std::vector<double> diag;     // per local row
-  // double-double factors: lo parts of val and diag (empty otherwise)
-  std::vector<double> val_lo;
-  std::vector<double> diag_lo;
-};
 
 // Level analysis.  forward: deps of row i are < i; backward: > i.
 void build_levels(BlockSweep& S, int nrow, bool forward) {
@@ -449,6 +436,22 @@ void pack_sweep(const std::vector<BlockSweep>& blocks, const std::vector<int>& b
   PARCEL_HIP_CHECK(hipStreamSynchronize(st));
 }
 
+// The counts pack_sweep reports, for sweeps whose level form is not built.
+void count_sweep(const std::vector<BlockSweep>& blocks, int padk, Sweep& S) {
+  long rows = 0, real = 0;
+  int nlev = 0;
+  for (const BlockSweep& B : blocks) {
+    if (!B.lev_start.empty()) nlev += (int)B.lev_start.size() - 1;
+    rows += (long)B.diag.size();
+    real += (long)B.dep.size();
+  }
+  if (rows * padk > 0x7fffffffL)
+    throw hip_error("block-Jacobi factor too large for int32 offsets", PARCEL_HIP_ERR_UNSUPPORTED);
+  S.nlev = nlev;
+  S.entries = rows * padk;
+  S.real_entries = real;
+}
+
 // --- kernels -----------------------------------------------------------------
 
 template <class T>
@@ -473,15 +476,6 @@ struct SweepArgs {
   int stride;
   int ldsbar;  // every dependency is in the LDS ring: level barriers need no HBM wait
 };
-
-// Barrier that orders LDS accesses only.  __syncthreads() also waits for
-// every outstanding global load and store of the wave (CDNA counts both in
-// vmcnt), which would drain the prefetch pipeline at every level.
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
 
 constexpr int kKR = 8;  // widest rows handled by the register-pipelined path
 
@@ -766,526 +760,6 @@ SweepArgs<float> sweep_args<float>(const Sweep& S) {
   return a;
 }
 
-// --- line-wavefront form of the FP64 apply ------------------------------------
-//
-// A block of P grid planes of ny lines of nx cells (P = 1: a strip of lines
-// of one plane, ny its line count) whose factor rows couple only to the cell
-// neighbour (offset 1), the line neighbour (offset nx) and the plane
-// neighbour (offset nx ny) is swept as a wavefront.  In sweep coordinates
-// (forward: cell i, line j, plane k; backward: nx-1-i, ny-1-j, P-1-k)
-// wavefront w = k WP + jw (WP = ceil(ny / 64) wavefronts per plane) owns
-// lines j = 64 jw + lane of plane k, and a thread computes cell
-// i = t - j - lag(w) at step t, lag(w) = 8 jw + 9 k.  Then the cell neighbour
-// was computed at step t-1 by the thread itself, the line neighbour at t-1 by
-// the lane below (a DPP wave shift) or, for lane 0, at t-9 by lane 63 of the
-// wavefront before (through an LDS line indexed by cell), and the plane
-// neighbour at t-9 by the same lane of wavefront w - WP (through an LDS ring
-// of the last kLR steps of every line).  One LDS barrier per kLG = 8 steps
-// publishes both: a value written at step t-9 or earlier was written in an
-// earlier group.  Every row sums its couplings in the stored order with the
-// same fma sequence as the level-scheduled kernels, so the values are
-// bit-identical to theirs.
-//
-// Memory: the rows of one step of a wavefront are one anti-diagonal of its
-// lines, nx - 1 apart in the natural order of the vectors.  The factor
-// arrays are stored per wavefront in anti-diagonal order (one coalesced load
-// per step); the vectors go through LDS in groups of kLG steps: each line of
-// a group is kLG consecutive cells, which the wavefront loads and stores as
-// 64-byte segments (lane 8j + c: line 8k + j, cell c, k = 0..7) and the
-// owning lane reads and writes in its slot row.  The fused update r -= alpha q
-// is elementwise and is applied (and stored) while a group's inputs are staged.
-constexpr int kLG = 8;
-static_assert(kLG == 8, "the staging moves 8 lines x 8 cells per instruction");
-constexpr int kLS = kLG + 1;  // doubles per line of a wavefront's slots (padding against bank conflicts)
-constexpr int kLPlag = kLG + 1;  // steps between a line and the same line of the next plane
-// Ring depth of the plane hand-over: the value of step s is read at s + 9, in
-// group floor((s + 9) / 8); it may be overwritten from the next group on,
-// at s + kLR >= 8 (floor((s + 9) / 8) + 1), which holds for every s at 17.
-constexpr int kLR = 17;
-
-// Entries on the anti-diagonals 0..d-1 of an nl x nx sub-block (anti-diagonal
-// d' holds min(d', nl-1) - max(0, d'-nx+1) + 1 cells); the cell of line l on
-// anti-diagonal d sits at line_doff(d) + l - max(0, d - nx + 1).
-__host__ __device__ inline long line_doff(int d, int nl, int nx) {
-  const long a = d < nl ? d : nl;
-  const long over = d > nx ? d - nx : 0;
-  return a * (a + 1) / 2 + (long)(d > nl ? d - nl : 0) * nl - over * (over + 1) / 2;
-}
-
-struct LineArgs {
-  const int* bstart;
-  const double* fc;  // per row: line and cell couplings, in the sweep's stored order
-  const double* fp;  // per row: plane coupling (P > 1)
-  const double* fd;
-  const double* bc;
-  const double* bp;
-  const double* bd;
-  double* sink;  // 64 doubles per block: the stores of lanes off the block's cells
-  int nx;
-  int ny;        // lines per plane (0: every block is one plane of its own line count)
-};
-
-// v of the lane below (DPP wave_shr:1); lane 0 receives `first`.
-__device__ __forceinline__ double from_lane_below(double first, double v) {
-  const long long o = __double_as_longlong(first), x = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_update_dpp((int)o, (int)x, 0x138, 0xf, 0xf, false);
-  const int hi = __builtin_amdgcn_update_dpp((int)(o >> 32), (int)(x >> 32), 0x138, 0xf, 0xf, false);
-  return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
-}
-
-// Orders the LDS accesses of the lanes of one wavefront (no s_barrier: the
-// slots are private to the wavefront).
-__device__ __forceinline__ void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
-}
-
-// Factor operands of one step, loaded kLG steps ahead.
-struct LineOps {
-  double c0, c1;  // the row's line and cell couplings in stored order
-  double cp;      // plane coupling
-  double d;       // scale
-};
-
-// The couplings' stored order is fixed by the factor: the forward rows of
-// both factors and the backward rows of D-ILU hold the plane neighbour
-// first, then the line neighbour, then the cell neighbour (ILU(0) keeps the
-// CRS order of the block, D-ILU walks its upper part downward); ILU(0)'s
-// backward rows hold them the other way round.
-template <bool FWD, int MODE>
-constexpr bool line_cell_first() { return !FWD && MODE == BJ_ILU0; }
-
-// Blocks of one plane with at most four wavefronts stage through a 16-cell
-// ring per line instead (kLA doubles with padding): each group loads one
-// aligned 8-cell chunk of every line and stores its newest complete one, so
-// the vector traffic moves whole 64-byte sectors when lines start on one.
-// Row stride 20 doubles (16 ring cells, padding slot 16): a step's lanes read
-// cell (a - lane) mod 16 of their rows, which at this stride fall in distinct
-// banks (at 17 they would all share a bank pair).
-constexpr int kLA = 20;
-__host__ __device__ constexpr bool line_aligned(bool planes, int W) { return !planes && W <= 4; }
-
-// Dynamic LDS of k_bj_lines, in doubles: slots, line hand-over, plane ring.
-__host__ __device__ inline size_t line_lds_doubles(int W, int nx, int planes) {
-  const size_t slots = (size_t)64 * W * (line_aligned(planes > 1, W) ? kLA : kLS);
-  return slots + (size_t)W * nx + (planes > 1 ? (size_t)64 * W * kLR : 0);
-}
-
-template <bool FWD, int MODE, bool FUSED, bool PL, int W>
-__device__ __forceinline__ void line_sweep(const LineArgs& A, int lo, int ny, int np, const double* rin,
-                                           double* s, const double* q, double* rout, double alpha,
-                                           double* lds) {
-  constexpr bool kScale = !(FWD && MODE == BJ_ILU0);
-  constexpr bool kCellFirst = line_cell_first<FWD, MODE>();
-  const int nx = A.nx;
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int WP = (ny + 63) >> 6;             // wavefronts per plane
-  const int kp = w / WP, jw = w - kp * WP;   // this wavefront's plane and line group
-  const bool wact = kp < np;                 // the others idle through the barriers
-  const int j = 64 * jw + lane;
-  const bool lact = wact && j < ny;
-  const int nlw = wact ? min(64, ny - 64 * jw) : 1;  // lines of this wavefront
-  const int lag = 8 * jw + kLPlag * kp;
-  const int nsteps = nx + ny - 1 + 8 * (WP - 1) + kLPlag * (np - 1);
-  const double* cc = FWD ? A.fc : A.bc;
-  const double* cpl = FWD ? A.fp : A.bp;
-  const double* dv = FWD ? A.fd : A.bd;
-  double* sink = A.sink + (long)blockIdx.x * 64 + lane;
-  // sweep line (j, kp) -> first row of the line; the wavefront's sub-block of entries
-  auto line_row = [&](int jj) -> int {
-    return lo + ((FWD ? kp : np - 1 - kp) * ny + (FWD ? jj : ny - 1 - jj)) * nx;
-  };
-  const long sub = (long)lo + (long)(kp * ny + 64 * jw) * nx;
-  constexpr bool ALN = line_aligned(PL, W);
-  constexpr int kSL = ALN ? kLA : kLS;
-  double* ws = lds + w * 64 * kSL;  // this wavefront's slots: [line][step of the group] / [line][cell mod 16]
-  double* my = ws + lane * kSL;
-  double* hand = lds + 64 * W * kSL;  // [wavefront][cell]: lane 63's values
-  double* ring = hand + W * nx;       // [thread][step mod kLR]: every line's values (P > 1)
-  // staging lanes: lane 8j + c moves cell c of the group for local line 8k + j;
-  // rows of the current group (stores) and of the next (loads), -1 off the block
-  const int sj = lane >> 3, sc = lane & 7;
-  int rcur[8], rnext[8], cnext[8];
-  // cells t1 - j - lag + 0..7 of the group starting at step t1 (ALN = false)
-  auto stage_rows = [&](int t1, int off) {
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      const int jj = 64 * jw + 8 * k + sj;
-      const int ip = t1 + off + sc - jj - lag;
-      const bool v = wact && jj < ny && (unsigned)ip < (unsigned)nx;
-      rnext[k] = v ? line_row(jj) + (FWD ? ip : nx - 1 - ip) : -1;
-      cnext[k] = ip;
-    }
-  };
-  // ALN: the chunk cells advance by exactly 8 per group, so each staging lane
-  // carries the cell of its input chunk (loaded during a group for the next)
-  // and of its output chunk (stored after a group) and the first row of its
-  // line (backward: the row of cell 0, rows descending)
-  int lrow[8], cin[8], cout[8];
-  bool lv[8];
-  if (ALN) {
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      const int jj = 64 * jw + 8 * k + sj;
-      const int a0 = -jj - lag;  // the line's cell at step 0
-      lv[k] = wact && jj < ny;
-      lrow[k] = line_row(min(jj, ny - 1)) + (FWD ? 0 : nx - 1);
-      cout[k] = ((a0 >> 3) << 3) + sc;
-      cin[k] = (((a0 + 15) >> 3) << 3) + sc;
-    }
-  }
-  auto chunk_rows = [&](const int (&cell)[8], bool first) {
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      const int jj = 64 * jw + 8 * k + sj;
-      const bool v = lv[k] && (unsigned)cell[k] < (unsigned)nx && !(first && ((-jj - lag) & 7) == 0);
-      rnext[k] = v ? (FWD ? lrow[k] + cell[k] : lrow[k] - cell[k]) : -1;
-      cnext[k] = cell[k];
-    }
-  };
-  double va[8], vb[8];
-  auto stage_load = [&]() {
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      const long row = rnext[k] >= 0 ? rnext[k] : lo;
-      va[k] = FWD ? rin[row] : s[row];
-      if (FUSED) vb[k] = q[row];
-    }
-  };
-  auto stage_fill = [&]() {
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      double z0 = va[k];
-      if (FUSED) {
-        z0 = fma(-alpha, vb[k], va[k]);
-        *(rnext[k] >= 0 ? rout + rnext[k] : sink) = z0;
-      }
-      // aligned ring: cells off the block go to the padding slot 16
-      ws[(8 * k + sj) * kSL + (ALN ? (rnext[k] >= 0 ? (cnext[k] & 15) : 16) : sc)] = z0;
-      rcur[k] = rnext[k];
-    }
-  };
-  auto stage_store = [&]() {
-#pragma unroll
-    for (int k = 0; k < 8; ++k)
-      *(rcur[k] >= 0 ? s + rcur[k] : sink) = ws[(8 * k + sj) * kSL + (ALN ? (cnext[k] & 15) : sc)];
-  };
-  // factor loads: anti-diagonal dl = t - lag - 64 jw of the wavefront's own
-  // lines for the next load and the entry offset of its line 0 on it
-  // (wave-uniform, advanced one step per load)
-  int dl = -lag - 64 * jw;
-  long offl = 0;
-  auto load = [&](int t, LineOps& o) {
-    const int ip = t - j - lag;
-    const bool on = lact && (unsigned)ip < (unsigned)nx;
-    const long e = on ? sub + offl + lane : (long)lo;
-    const double2 cv = reinterpret_cast<const double2*>(cc)[e];
-    o.c0 = cv.x;
-    o.c1 = cv.y;
-    if (PL) o.cp = cpl[e];
-    if (kScale) o.d = dv[e];
-    if (dl >= 0) offl += min(dl, nlw - 1) - max(0, dl - nx + 1) + 1 - (dl >= nx - 1 ? 1 : 0);
-    ++dl;
-  };
-  // An absent coupling has coefficient +0 and neighbour value kZero, whose
-  // product term is -0 in the row's fma (fma(-(+0), +0, z) forward and in
-  // ILU(0)'s backward rows, fma(-0, +0, z) in D-ILU's), and z + (-0) == z for
-  // every z, the signed zeros included: the same bits as skipping the term.
-  // The values start as kZero (the cell before a line's first, the line below
-  // a plane's first, the plane below the block's first).
-  constexpr double kZero = (!FWD && MODE == BJ_DILU) ? -0.0 : 0.0;
-  double yprev = kZero;  // the thread's value of the previous step (its cell neighbour)
-  auto step = [&](int t, double a, double hv, double pv, const LineOps& o) -> double {
-    const int ip = t - j - lag;
-    const bool on = lact && (unsigned)ip < (unsigned)nx;
-    const double yd = from_lane_below(hv, yprev);  // line neighbour
-    double y;
-    if (!FWD && MODE == BJ_DILU) {
-      // plane, line, cell; y = a - d * sum
-      double z = PL ? fma(pv, o.cp, 0.0) : fma(yd, o.c0, 0.0);
-      z = PL ? fma(yd, o.c0, z) : z;
-      z = fma(yprev, o.c1, z);
-      y = fma(-o.d, z, a);
-    } else if (kCellFirst) {
-      double z = fma(-yprev, o.c0, a);
-      z = fma(-yd, o.c1, z);
-      if (PL) z = fma(-pv, o.cp, z);
-      y = z / o.d;
-    } else {
-      double z = PL ? fma(-pv, o.cp, a) : a;
-      z = fma(-yd, o.c0, z);
-      z = fma(-yprev, o.c1, z);
-      y = MODE == BJ_ILU0 ? z : o.d * z;
-    }
-    if (W > 1 && lane == 63 && jw < WP - 1 && on) hand[w * nx + ip] = y;
-    if (PL) ring[tid * kLR + t % kLR] = y;
-    yprev = on ? y : yprev;
-    return y;
-  };
-  LineOps R[kLG];
-  // one group of kLG steps: the next group's vectors are in flight during it
-  auto group = [&](int t0) {
-    if (ALN) chunk_rows(cin, false);
-    else stage_rows(t0 + kLG, 0);
-    stage_load();
-    wave_lds_sync();
-    // the group's inputs and hand-over values, read before its first step
-    // (the hand-over values were written in earlier groups)
-    double av[kLG], hv[kLG], pv[kLG];
-#pragma unroll
-    for (int u = 0; u < kLG; ++u) {
-      av[u] = my[ALN ? ((t0 + u - j - lag) & 15) : u];
-      const int ip = min(max(t0 + u - j - lag, 0), nx - 1);
-      hv[u] = (W > 1 && jw > 0) ? hand[(w - 1) * nx + ip] : kZero;
-      if (PL) pv[u] = (kp > 0) ? ring[(tid - 64 * WP) * kLR + (t0 + u + kLR - kLPlag) % kLR] : kZero;
-    }
-#pragma unroll
-    for (int u = 0; u < kLG; ++u) {
-      const int ip = t0 + u - j - lag;
-      const bool on = lact && (unsigned)ip < (unsigned)nx;
-      my[ALN ? (on ? (ip & 15) : 16) : u] = step(t0 + u, av[u], hv[u], PL ? pv[u] : kZero, R[u]);
-      load(t0 + u + kLG, R[u]);
-    }
-    wave_lds_sync();
-    if (ALN) {
-      // the newest complete chunk of every line: its cells were the ring's
-      // since the group before (in-place: input, then the row's value)
-      const int rl[8] = {rnext[0], rnext[1], rnext[2], rnext[3], rnext[4], rnext[5], rnext[6], rnext[7]};
-      const int cl[8] = {cnext[0], cnext[1], cnext[2], cnext[3], cnext[4], cnext[5], cnext[6], cnext[7]};
-      chunk_rows(cout, false);
-#pragma unroll
-      for (int k = 0; k < 8; ++k) rcur[k] = rnext[k];
-      stage_store();
-#pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        rnext[k] = rl[k];
-        cnext[k] = cl[k];
-        cin[k] += kLG;
-        cout[k] += kLG;
-      }
-    } else {
-      stage_store();
-    }
-    wave_lds_sync();
-    stage_fill();
-    if (W > 1) lds_barrier();
-  };
-  if (ALN) {
-    // the chunks group 0 reads: cells a .. a + 7 of every line lie in chunks
-    // a >> 3 (cout's) and (a + 7) >> 3 (cin's minus one)
-    chunk_rows(cout, true);
-    stage_load();
-    stage_fill();
-    wave_lds_sync();
-    int c1[8];
-#pragma unroll
-    for (int k = 0; k < 8; ++k) c1[k] = cin[k] - kLG;
-    chunk_rows(c1, false);
-  } else {
-    stage_rows(0, 0);
-  }
-  stage_load();
-  stage_fill();
-#pragma unroll
-  for (int u = 0; u < kLG; ++u) load(u, R[u]);
-  // the first group runs outside the loop, so that the loop is entered with
-  // the memory operations of a whole group in flight on both of its paths
-  // (the compiler's wait counts then match the steady state); with aligned
-  // chunks one more group stores the lines' last chunks
-  group(0);
-  for (int t0 = kLG; t0 < nsteps + (ALN ? kLG - 1 : 0); t0 += kLG) group(t0);
-}
-
-// One workgroup of 64 W threads per block: forward then backward sweep.  The
-// fused residual update computes alpha as k_bj_apply does, with gamma summed
-// in the same order (partials j, j + kNT, ... per virtual thread j < kNT,
-// wavefront sums, then the kWaves sums in order).
-template <int MODE, int W, bool PL>
-__global__ void __launch_bounds__(64 * W) k_bj_lines(LineArgs A, const double* rin, double* s, CGFuse fuse,
-                                                     const int* skip) {
-  if (skip && *skip) return;
-  extern __shared__ double lds_lines[];
-  __shared__ double sh[kWaves];
-  double alpha = 0.0;
-  const double* q = nullptr;
-  double* rout = nullptr;
-  if (fuse.st) {
-    const int d = fuse.st->done_at;
-    if (d != 0 && d <= fuse.it) return;
-    CGSlot* sl = &fuse.st->slot[fuse.it & 1];
-    for (int vw = threadIdx.x >> 6; vw < kWaves; vw += W) {
-      double a = 0.0;
-      for (int j = vw * 64 + (threadIdx.x & 63); j < fuse.nb_prod; j += kNT) a = a + fuse.part_gamma[j];
-      a = wave_sum(a);
-      if ((threadIdx.x & 63) == 0) sh[vw] = a;
-    }
-    __syncthreads();
-    double gamma = sh[0];
-    for (int k = 1; k < kWaves; ++k) gamma = gamma + sh[k];
-    alpha = sl->rho0 / gamma;
-    if (blockIdx.x == 0 && threadIdx.x == 0) sl->alpha = alpha;
-    q = fuse.q;
-    rout = fuse.r;
-    rin = fuse.r;
-  }
-  const int lo = A.bstart[blockIdx.x];
-  const int lines = (A.bstart[blockIdx.x + 1] - lo) / A.nx;
-  const int ny = A.ny > 0 ? A.ny : lines;
-  const int np = lines / ny;
-  if (q) line_sweep<true, MODE, true, PL, W>(A, lo, ny, np, rin, s, q, rout, alpha, lds_lines);
-  else line_sweep<true, MODE, false, PL, W>(A, lo, ny, np, rin, s, nullptr, nullptr, 0.0, lds_lines);
-  __syncthreads();  // forward values in memory before other threads' backward rows read them
-  line_sweep<false, MODE, false, PL, W>(A, lo, ny, np, nullptr, s, nullptr, nullptr, 0.0, lds_lines);
-}
-
-constexpr size_t kLineLdsMax = 64 * 1024 - 64;  // dynamic LDS of k_bj_lines
-
-// Set up the line-wavefront form when the block factors have its pattern
-// (FP64 applies only; the level-scheduled sweeps stay for the other paths).
-// PARCEL_HIP_BJ_LEVELS=1 in the environment keeps the level-scheduled apply.
-bool line_setup(Plan& P, const std::vector<BlockSweep>& F, const std::vector<BlockSweep>& B,
-                const std::vector<int>& blo, const std::vector<int>& bhi) {
-  Precon& M = P.M;
-  LineBJ& G = M.line;
-  G = LineBJ();
-  if (const char* e = std::getenv("PARCEL_HIP_BJ_LEVELS"))
-    if (e[0] && e[0] != '0') return false;
-  const int n = P.hA.n, nblk = (int)F.size();
-  // the forward dependency offsets above 1: nx, and nx ny when blocks hold several planes
-  long nx = 0, nxy = 0;
-  for (int b = 0; b < nblk; ++b)
-    for (size_t i = 0; i + 1 < F[b].ptr.size(); ++i)
-      for (int q = F[b].ptr[i]; q < F[b].ptr[i + 1]; ++q) {
-        const long off = (long)i - F[b].dep[q];
-        if (off <= 1 || off == nx || off == nxy) continue;
-        if (!nx) nx = off;
-        else if (!nxy) nxy = off;
-        else return false;
-      }
-  if (nx && nxy && nxy < nx) std::swap(nx, nxy);
-  if (nx < 2 || (nxy && nxy % nx)) return false;
-  const int X = (int)nx;
-  const int NY = nxy ? (int)(nxy / nx) : 0;  // lines per plane (0: one plane per block)
-  for (int b = 0; b + 1 < nblk; ++b)
-    if (bhi[b] != blo[b + 1]) return false;
-  int W = 1, np_max = 1;
-  for (int b = 0; b < nblk; ++b) {
-    const long len = (long)bhi[b] - blo[b];
-    const long unit = nxy ? nxy : nx;
-    if (len <= 0 || blo[b] % unit || len % unit) return false;
-    const int lines = (int)(len / nx), ny = NY ? NY : lines, np = lines / ny;
-    const int waves = ((ny + 63) / 64) * np;
-    if (waves > 8) return false;
-    while (W < waves) W *= 2;
-    np_max = std::max(np_max, np);
-  }
-  const bool PL = np_max > 1;
-  if (sizeof(double) * line_lds_doubles(W, X, np_max) > kLineLdsMax || (PL && W > 4)) return false;
-  const bool ilu0 = M.mode == BJ_ILU0;
-  std::vector<double> fc(2 * (size_t)n, 0.0), bc(2 * (size_t)n, 0.0), fd(n, 0.0), bd(n, 0.0);
-  std::vector<double> fp(PL ? n : 0, 0.0), bp(PL ? n : 0, 0.0);
-  int bad = 0;
-#pragma omp parallel for schedule(dynamic) reduction(| : bad)
-  for (int b = 0; b < nblk; ++b) {
-    const int lo = blo[b], lines = (bhi[b] - lo) / X, ny = NY ? NY : lines, np = lines / ny;
-    for (int k = 0; k < np && !bad; ++k)
-      for (int jj = 0; jj < ny && !bad; ++jj)
-        for (int x = 0; x < X; ++x) {
-          const int i = (k * ny + jj) * X + x;  // local row
-          for (int dir = 0; dir < 2; ++dir) {
-            const BlockSweep& S = dir == 0 ? F[b] : B[b];
-            const bool fwd = dir == 0;
-            // the neighbours the sweep reads, in the kernel's order
-            const int cn = fwd ? i - 1 : i + 1, ln = fwd ? i - X : i + X, pn = fwd ? i - X * ny : i + X * ny;
-            const bool hc = fwd ? x > 0 : x < X - 1, hl = fwd ? jj > 0 : jj < ny - 1, hp = fwd ? k > 0 : k < np - 1;
-            const bool cell_first = !fwd && ilu0;
-            int want[3], nw = 0;
-            if (cell_first) {
-              if (hc) want[nw++] = cn;
-              if (hl) want[nw++] = ln;
-              if (hp) want[nw++] = pn;
-            } else {
-              if (hp) want[nw++] = pn;
-              if (hl) want[nw++] = ln;
-              if (hc) want[nw++] = cn;
-            }
-            if (S.ptr[i + 1] - S.ptr[i] != nw) { bad = 1; break; }
-            double vc = 0.0, vl = 0.0, vp = 0.0;
-            for (int q = S.ptr[i], m = 0; q < S.ptr[i + 1]; ++q, ++m) {
-              const int dp = S.dep[q];
-              if (dp != want[m]) { bad = 1; break; }
-              (dp == cn ? vc : dp == ln ? vl : vp) = S.val[q];
-            }
-            if (bad) break;
-            // sweep coordinates, the wavefront's sub-block and its anti-diagonal entry
-            const int ip = fwd ? x : X - 1 - x, jp = fwd ? jj : ny - 1 - jj, kq = fwd ? k : np - 1 - k;
-            const int jw = jp / 64, l = jp % 64, nlw = std::min(64, ny - 64 * jw), dg = ip + l;
-            const long e = (long)lo + (long)(kq * ny + 64 * jw) * X + line_doff(dg, nlw, X) + l -
-                           std::max(0, dg - X + 1);
-            std::vector<double>& cv = fwd ? fc : bc;
-            cv[2 * (size_t)e] = cell_first ? vc : vl;
-            cv[2 * (size_t)e + 1] = cell_first ? vl : vc;
-            if (PL) (fwd ? fp : bp)[(size_t)e] = vp;
-            (fwd ? fd : bd)[(size_t)e] = S.diag[i];
-          }
-          if (bad) break;
-        }
-  }
-  if (bad) return false;
-  std::vector<int> bs(nblk + 1);
-  for (int b = 0; b < nblk; ++b) bs[b] = blo[b];
-  bs[nblk] = bhi[nblk - 1];
-  G.bstart.upload(bs, P.stream);
-  G.fc.upload(fc, P.stream);
-  G.bc.upload(bc, P.stream);
-  G.fd.upload(fd, P.stream);
-  G.bd.upload(bd, P.stream);
-  if (PL) {
-    G.fp.upload(fp, P.stream);
-    G.bp.upload(bp, P.stream);
-  }
-  G.sink.alloc((size_t)64 * nblk);
-  PARCEL_HIP_CHECK(hipStreamSynchronize(P.stream));
-  G.nx = X;
-  G.ny = NY;
-  G.planes = np_max;
-  G.waves = W;
-  G.on = true;
-  return true;
-}
-
-void line_apply(Plan& P, const double* r, double* s, const CGFuse* fuse, const int* skip) {
-  const Precon& M = P.M;
-  const LineBJ& G = M.line;
-  LineArgs A{G.bstart.p, G.fc.p, G.fp.p, G.fd.p, G.bc.p, G.bp.p, G.bd.p, G.sink.p, G.nx, G.ny};
-  CGFuse f;
-  if (fuse) f = *fuse;
-  const size_t shm = sizeof(double) * line_lds_doubles(G.waves, G.nx, G.planes);
-  const dim3 grid(M.nblocks);
-#define PARCEL_LINE_K(W, PL)                                                                                    \
-  do {                                                                                                          \
-    if (M.mode == BJ_ILU0)                                                                                      \
-      hipLaunchKernelGGL((k_bj_lines<BJ_ILU0, W, PL>), grid, dim3(64 * W), shm, P.stream, A, r, s, f, skip);   \
-    else                                                                                                        \
-      hipLaunchKernelGGL((k_bj_lines<BJ_DILU, W, PL>), grid, dim3(64 * W), shm, P.stream, A, r, s, f, skip);   \
-  } while (0)
-  if (G.planes > 1) {
-    // eight wavefronts with the plane ring exceed the LDS budget (line_setup)
-    if (G.waves == 2) PARCEL_LINE_K(2, true);
-    else PARCEL_LINE_K(4, true);
-  } else {
-    switch (G.waves) {
-      case 1: PARCEL_LINE_K(1, false); break;
-      case 2: PARCEL_LINE_K(2, false); break;
-      case 4: PARCEL_LINE_K(4, false); break;
-      default: PARCEL_LINE_K(8, false); break;
-    }
-  }
-#undef PARCEL_LINE_K
-}
-
 // Line-scan form of the FP32 inner apply (mixed-precision solver): when every
 // block-Jacobi block is a strip of whole grid lines of one nx-cell line
 // length, the strips are the equal split [ny k / nblk, ny (k+1) / nblk) of
@@ -1439,10 +913,14 @@ void precon_setup(Plan& P) {
         for (size_t l = 0; l + 1 < S->lev_start.size(); ++l)
           maxw = std::max(maxw, S->lev_start[l + 1] - S->lev_start[l]);
     M.nth = maxw <= 256 ? 256 : maxw <= 512 ? 512 : 1024;
-    pack_sweep(F, blo, M.fwd, kRingBudget, apply_k(kmax), M.nth, P.stream);
-    pack_sweep(B, blo, M.bwd, kRingBudget, apply_k(kmax), M.nth, P.stream);
-    lscan_setup(P, F, B, blo, bhi);
-    if (P.prm.solver != PARCEL_SOLVER_CG_MIXED) line_setup(P, F, B, blo, bhi);
+    if (P.prm.solver != PARCEL_SOLVER_CG_MIXED && line_setup(P, F, B, blo, bhi, 1)) {
+      count_sweep(F, apply_k(kmax), M.fwd);
+      count_sweep(B, apply_k(kmax), M.bwd);
+    } else {
+      pack_sweep(F, blo, M.fwd, kRingBudget, apply_k(kmax), M.nth, P.stream);
+      pack_sweep(B, blo, M.bwd, kRingBudget, apply_k(kmax), M.nth, P.stream);
+      lscan_setup(P, F, B, blo, bhi);
+    }
   } else if (M.kind != PRECON_NONE) {
     throw hip_error("preconditioner not supported on this path", PARCEL_HIP_ERR_UNSUPPORTED);
   }

@@ -179,7 +179,7 @@ def test_mpnn_training_lowers_loss():
 
 @pytest.mark.parametrize("nx,ny", [(33, 31), (512, 40)])
 def test_mpnn_gradients_partial_counts(nx, ny):
-    # 256 and 1280 per-wavefront partials: the remainder loop of the sum over
+    # 64 and 1280 per-wavefront partials: the remainder loop of the sum over
     # partials alone, and its unrolled rounds followed by a remainder; the
     # bound is the BF16 one of the gradients
     test_mpnn_gradients_match_oracle(nx, ny)
