@@ -176,11 +176,11 @@ constexpr bool line_cell_first() { return !FWD && MODE == BJ_ILU0; }
 
 // dd_div(z, 1) for the unit pivots of ILU(0)'s forward rows: with d = 1 the
 // quotient's q1 is z.hi, its remainder 0 + z.lo and q2 that, so the result
-// is z's parts added and split again (the same bits, finite z).  dd_div's
-// split product overflows beyond 2^996 and for non-finite z: those take it.
-__device__ __forceinline__ dd dd_div_one(dd z) {
-  if (!(fabs(z.hi) < 0x1p990)) return dd_div(z, mkdd(1.0, 0.0));
-  const double l = 0.0 + z.lo;
+// is z's parts added and split again (the same bits).  nan is 0, or NaN where
+// dd_div's split of q1 overflows (|z.hi| beyond 2^996 or not finite).
+__host__ __device__ __forceinline__ dd dd_div_one(dd z) {
+  const double nan = 0.0 * (134217729.0 * z.hi);
+  const double l = (0.0 + z.lo) + nan;
   const double h = z.hi + l;
   return mkdd(h, l - (h - z.hi));
 }
@@ -364,18 +364,23 @@ __device__ __forceinline__ void line_sweep(const LineArgs& A, const LineBlock bk
     // in(g + 1)
     stage_load(Q{}, ri, ci);
     wave_lds_sync();
-    V av[kLG], hv[kLG], pv[kLG];
+    auto input = [&](int u, V& a, V& h, V& pl) {
+      a = N::get(own[s0 + u]);
+      if (MULTI) h = N::get(u > 0 ? hnd[s1 + u - 1] : hnd[s2 + 7]);
+      if (PL) pl = N::get(u > 0 ? pln[s1 + u - 1] : pln[s2 + 7]);
+    };
+    // all of the group's inputs at its start; double-double (twice the
+    // registers, and steps longer than an LDS round trip) one step ahead
+    constexpr int NI = NV == 1 ? kLG : 2;
+    V av[NI], hv[NI], pv[NI];
+#pragma unroll
+    for (int u = 0; u < NI; ++u) hv[u] = pv[u] = N::num(kZero);
+#pragma unroll
+    for (int u = 0; u < (NV == 1 ? kLG : 1); ++u) input(u, av[u], hv[u], pv[u]);
 #pragma unroll
     for (int u = 0; u < kLG; ++u) {
-      av[u] = N::get(own[s0 + u]);
-      hv[u] = N::num(kZero);
-      pv[u] = N::num(kZero);
-      if (MULTI) hv[u] = N::get(u > 0 ? hnd[s1 + u - 1] : hnd[s2 + 7]);
-      if (PL) pv[u] = N::get(u > 0 ? pln[s1 + u - 1] : pln[s2 + 7]);
-    }
-#pragma unroll
-    for (int u = 0; u < kLG; ++u) {
-      own[s0 + u] = N::put(step(u, av[u], hv[u], pv[u], R[(p * kLG + u) % NR]));
+      if (NV == 2 && u + 1 < kLG) input(u + 1, av[(u + 1) % NI], hv[(u + 1) % NI], pv[(u + 1) % NI]);
+      own[s0 + u] = N::put(step(u, av[u % NI], hv[u % NI], pv[u % NI], R[(p * kLG + u) % NR]));
       load(u + NR, R[(p * kLG + u) % NR]);
     }
     wave_lds_sync();
@@ -754,6 +759,31 @@ void line_apply(Plan& P, const double* r, double* s, const CGFuse* fuse, const i
 #undef PARCEL_LINE_W
 #undef PARCEL_LINE_P
 #undef PARCEL_LINE_F
+}
+
+void line_apply_dd(Plan& P, const double* rh, const double* rl, double* sh, double* sl, const int* skip) {
+  const Precon& M = P.M;
+  const LineBJ& G = M.line;
+  const LineArgs A = line_args(G);
+  const size_t shm = line_lds_bytes(G.waves, 2);
+#define PARCEL_LINE_K(MODE, NTH, PL) \
+  launch_lines(k_bj_lines_dd<MODE, NTH, PL>, M.nblocks, G.waves, shm, P.stream, A, rh, rl, sh, sl, skip)
+#define PARCEL_LINE_P(MODE, NTH)               \
+  do {                                         \
+    if (G.nxy) PARCEL_LINE_K(MODE, NTH, true); \
+    else PARCEL_LINE_K(MODE, NTH, false);      \
+  } while (0)
+#define PARCEL_LINE_W(MODE)                           \
+  do {                                                \
+    if (G.waves == 1) PARCEL_LINE_K(MODE, 64, false); \
+    else if (G.waves <= 4) PARCEL_LINE_P(MODE, 256);  \
+    else PARCEL_LINE_P(MODE, 512);                    \
+  } while (0)
+  if (M.mode == BJ_ILU0) PARCEL_LINE_W(BJ_ILU0);
+  else PARCEL_LINE_W(BJ_DILU);
+#undef PARCEL_LINE_W
+#undef PARCEL_LINE_P
+#undef PARCEL_LINE_K
 }
 
 }  // namespace parcel

@@ -1334,21 +1334,27 @@ void precon_setup_dd(Plan& P, int prec) {
       for (const BlockSweep* S : {&F[b], &B[b]})
         for (size_t l = 0; l + 1 < S->lev_start.size(); ++l)
           maxw = std::max(maxw, S->lev_start[l + 1] - S->lev_start[l]);
-    // the pipelined kernel (k_dd_bj_fast) when every level fits 256 or 512
+    // line wavefronts (bjlines.hip) when the blocks have their pattern; else the
+    // pipelined level kernel (k_dd_bj_fast) when every level fits 256 or 512
     // threads, rows have at most kKR entries and both sweeps keep their
     // dependencies in the LDS ring; otherwise global row ids for k_dd_bj
     const int kk = apply_k(kmax);
     M.nth = maxw <= 256 ? 256 : 512;
     bool fast = maxw <= 512 && kk <= kKR;
-    if (fast) {
-      pack_sweep(F, blo, M.fwd, kRingBudget, kk, M.nth, P.stream);
-      pack_sweep(B, blo, M.bwd, kRingBudget, kk, M.nth, P.stream);
-      fast = M.fwd.ring > 0 && M.bwd.ring > 0;
-    }
-    if (!fast) {
-      M.nth = 256;
-      pack_sweep(F, blo, M.fwd, 0, kmax, M.nth, P.stream);
-      pack_sweep(B, blo, M.bwd, 0, kmax, M.nth, P.stream);
+    if (line_setup(P, F, B, blo, bhi, 2)) {
+      count_sweep(F, fast ? kk : kmax, M.fwd);
+      count_sweep(B, fast ? kk : kmax, M.bwd);
+    } else {
+      if (fast) {
+        pack_sweep(F, blo, M.fwd, kRingBudget, kk, M.nth, P.stream);
+        pack_sweep(B, blo, M.bwd, kRingBudget, kk, M.nth, P.stream);
+        fast = M.fwd.ring > 0 && M.bwd.ring > 0;
+      }
+      if (!fast) {
+        M.nth = 256;
+        pack_sweep(F, blo, M.fwd, 0, kmax, M.nth, P.stream);
+        pack_sweep(B, blo, M.bwd, 0, kmax, M.nth, P.stream);
+      }
     }
   } else if (M.kind != PRECON_NONE) {
     throw hip_error("preconditioner not supported on the double-double path", PARCEL_HIP_ERR_UNSUPPORTED);
@@ -1364,6 +1370,8 @@ void precon_apply_dd(Plan& P, const double* rh, const double* rl, double* sh, do
     const bool pj = M.kind == PRECON_PJ;
     hipLaunchKernelGGL(k_dd_pj, dim3(tiled_nb(n)), dim3(kNT), 0, P.stream, n, rh, rl, pj ? (const double*)M.dinv.p : nullptr,
                        (pj && two) ? (const double*)M.dinv_lo.p : nullptr, sh, sl, skip);
+  } else if (M.line.on) {
+    line_apply_dd(P, rh, rl, sh, sl, skip);
   } else {
     const DDSweep F = dd_sweep(M.fwd), B = dd_sweep(M.bwd);
     if (M.fwd.ring > 0 && M.bwd.ring > 0) {

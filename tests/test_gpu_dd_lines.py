@@ -1,0 +1,49 @@
+"""The double-double block-Jacobi apply as line wavefronts (bjlines.hip)
+against the oracle's dd PCG, bit for bit: blocks of whole lines and planes
+and blocks that cut them, one, two and four to six wavefronts per block, the
+factor's lo parts used or not.  A few iterations reach every row."""
+import numpy as np
+import pytest
+
+import oracle as orc
+import parcel_hip as ph
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _init():
+    ph.init(0)
+
+
+CASES = {
+    "p2d_40x70_b3": (lambda: ph.poisson2d(40, 70, -1.0), 3),
+    "p3d_20_b20": (lambda: ph.poisson3d_spd(20, 20, 20), 20),
+    "p3d_13x11x9_b20": (lambda: ph.poisson3d_spd(13, 11, 9), 20),
+    "p3d_20_b7": (lambda: ph.poisson3d_spd(20, 20, 20), 7),
+    "diff_12x96x6_b2": (lambda: ph.diffusion3d(12, 96, 6, ph.loguniform(12 * 96 * 6, 5, 1e-4, 1e4)), 2),
+    "diff_17x70x5_b4": (lambda: ph.diffusion3d(17, 70, 5, ph.loguniform(17 * 70 * 5, 6, 1e-4, 1e4)), 4),
+}
+
+
+@pytest.mark.parametrize("ilu,pp", [(0, 2), (0, 1), (1, 2), (2, 1)])
+@pytest.mark.parametrize("case", sorted(CASES))
+def test_ddcg_bit_exact(case, ilu, pp):
+    gen, nb = CASES[case]
+    print("dd lines", case, ilu, pp, flush=True)
+    rp, col, val = gen()
+    n = rp.shape[0] - 1
+    b = ph.uniform(n, 91)
+    b[:: 6] = 0.0
+    b[1:: 9] = -0.0
+    blo = b * 2.0 ** -57
+    xh, xl = np.zeros(n), np.zeros(n)
+    hist, niter, iret = ph.ddcg(xh, xl, b, blo, rp, col, val, None, ipreflag=2, ILU_method=ilu, precon_thblock=nb,
+                                itrmax=25, rtolmax=1e-22, PRECISION_A=1, PRECISION_b=2, PRECISION_x=2,
+                                PRECISION_PRECONDITION=pp)
+    oh, ol, ho, no, io = orc.ddcg(rp, col, val, None, b, blo, ipreflag=2, ilu_method=ilu, nblocks=nb, prec=pp,
+                                  itrmax=25, rtol=1e-22)
+    assert (niter, iret) == (no, io)
+    assert np.array_equal(hist, ho)
+    assert np.array_equal(xh.view(np.uint64), oh.view(np.uint64))
+    assert np.array_equal(xl.view(np.uint64), ol.view(np.uint64))
