@@ -242,16 +242,97 @@ __global__ void __launch_bounds__(kNT) k_ca_qr_norm(int n, const double* __restr
     qi[j] = sc * vi[j];
 }
 
+// Sums over the 64 lanes of N values at once, each the xor butterfly's
+// (offsets 32..1, the same pairs, so the same bits), returned to every lane.
+// Both lanes of a pair add the same two numbers, so after a step half the
+// lanes are free: two values share one step (the half swaps of gfx950 for 32
+// and 16, a select and a row rotation for 8), and N values cost N / 2 + N / 4
+// + N / 8 additions before the last three steps instead of 6 N.
+template <int O>
+__device__ __forceinline__ double pair_step(double a, double b) {
+  // lanes with bit O clear end with a's step, the others with b's
+  const unsigned lane = threadIdx.x & 63;
+  if constexpr (O == 32 || O == 16) {
+    const unsigned long long ua = (unsigned long long)__double_as_longlong(a), ub = (unsigned long long)__double_as_longlong(b);
+    unsigned r0[2], r1[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const unsigned x = (unsigned)(ua >> (32 * h)), y = (unsigned)(ub >> (32 * h));
+      if constexpr (O == 32) {
+        const auto p = __builtin_amdgcn_permlane32_swap(x, y, false, false);
+        r0[h] = p[0];
+        r1[h] = p[1];
+      } else {
+        const auto p = __builtin_amdgcn_permlane16_swap(x, y, false, false);
+        r0[h] = p[0];
+        r1[h] = p[1];
+      }
+    }
+    return __longlong_as_double((long long)(((unsigned long long)r0[1] << 32) | r0[0])) +
+           __longlong_as_double((long long)(((unsigned long long)r1[1] << 32) | r1[0]));
+  } else {
+    const bool up = lane & O;
+    const double keep = up ? b : a, send = up ? a : b;
+    return keep + xor_lane<O>(send);
+  }
+}
+__device__ __forceinline__ double read_lane(double v, int lane) {
+  const unsigned long long u = (unsigned long long)__double_as_longlong(v);
+  const unsigned lo = __builtin_amdgcn_readlane((unsigned)u, lane), hi = __builtin_amdgcn_readlane((unsigned)(u >> 32), lane);
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+// The same for up to 64 values: N / 2 + N / 4 + ... additions.  Lane l ends
+// with the total of value sum_slot(l) (0 or undefined for slots from N on).
+__device__ __forceinline__ int sum_slot(int lane) { return (int)(__brev((unsigned)lane) >> 26); }
+template <int N, int O>
+__device__ __forceinline__ double wave_sum_lanes(const double* d) {
+  if constexpr (O == 0) return d[0];
+  constexpr int M = (N + 1) / 2;
+  double a[M];
+#pragma unroll
+  for (int k = 0; k < M; ++k) a[k] = pair_step<(O > 0 ? O : 1)>(d[2 * k], 2 * k + 1 < N ? d[2 * k + 1 < N ? 2 * k + 1 : 0] : 0.0);
+  return wave_sum_lanes<M, O / 2>(a);
+}
+
+// Values [0, N) of d, N <= 8: the total of value k ends in the lanes whose
+// bits 5, 4, 3 are k's bits 0, 1, 2.
+template <int N>
+__device__ __forceinline__ void wave_sum_n(double (&d)[N]) {
+  static_assert(N >= 1 && N <= 8, "eight values share the first three steps");
+  double a[4], b[2], c;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) a[k] = pair_step<32>(2 * k < N ? d[2 * k < N ? 2 * k : 0] : 0.0,
+                                                   2 * k + 1 < N ? d[2 * k + 1 < N ? 2 * k + 1 : 0] : 0.0);
+#pragma unroll
+  for (int k = 0; k < 2; ++k) b[k] = pair_step<16>(a[2 * k], a[2 * k + 1]);
+  c = pair_step<8>(b[0], b[1]);
+  c += xor_lane<4>(c);
+  c += xor_lane<2>(c);
+  c += xor_lane<1>(c);
+#pragma unroll
+  for (int k = 0; k < N; ++k) d[k] = read_lane(c, ((k & 1) << 5) | ((k & 2) << 3) | ((k & 4) << 1));
+}
+
 // ---- block CGS between blocks (t > 1) ------------------------------------
-// Partials of <Q_i, V_j> for Q columns i in [4*blockIdx.y, 4*blockIdx.y + 4)
-// (below c1) and the NV columns of V; slot i + c1*j.
+// Most Q columns per workgroup row of k_ca_bdots: V is read once per row, so
+// more columns mean fewer passes over V; QC * NV sums at most 64, what one
+// shared butterfly reduces (a second one and the registers cost more than the
+// pass saves).  NV = 9, c1 = 9, 17, 25 (mean), n = 2^21: 195 us with four
+// columns and a butterfly per sum, 160 us with four and shared butterflies,
+// 131 / 126 / 119 us with five / six / seven, 261 us with eight.
+constexpr int bdots_cols(int nv) { return 64 / nv < 8 ? 64 / nv : 8; }
+
+// Partials of <Q_i, V_j> for this workgroup row's share of the c1 Q columns
+// (at most QC) and the NV columns of V; slot i + c1*j.
 template <int NV>
-__global__ void __launch_bounds__(kNT) k_ca_bdots(int n, const double* Q, long ldq, int c1, const double* V,
-                                                  long ldv, double* part) {
-  constexpr int NP = 4 * NV;
+__global__ void __launch_bounds__(kNT) k_ca_bdots(int n, const double* __restrict__ Q, long ldq, int c1,
+                                                  const double* __restrict__ V, long ldv, double* part) {
+  constexpr int QC = bdots_cols(NV);
+  constexpr int NP = QC * NV;
   __shared__ double sh[kWaves * NP];
-  const int i0 = blockIdx.y * 4;
-  const int ni = (c1 - i0) < 4 ? (c1 - i0) : 4;
+  // the columns split evenly over the rows
+  const int i0 = (int)((long)c1 * blockIdx.y / gridDim.y);
+  const int ni = (int)((long)c1 * (blockIdx.y + 1) / gridDim.y) - i0;
   const int nb = gridDim.x;
   const long ntiles = ((long)n + kNT - 1) / kNT;
   double acc[NP];
@@ -260,25 +341,22 @@ __global__ void __launch_bounds__(kNT) k_ca_bdots(int n, const double* Q, long l
   for (long t = blockIdx.x; t < ntiles; t += nb) {
     const long q = t * kNT + threadIdx.x;
     if (q < n) {
-      double v[NV];
+      double v[NV], qv[QC];
+#pragma unroll
+      for (int ii = 0; ii < QC; ++ii) qv[ii] = Q[(long)(i0 + (ii < ni ? ii : 0)) * ldq + q];
 #pragma unroll
       for (int j = 0; j < NV; ++j) v[j] = V[(long)j * ldv + q];
 #pragma unroll
-      for (int ii = 0; ii < 4; ++ii) {
-        if (ii < ni) {
-          const double qv = Q[(long)(i0 + ii) * ldq + q];
+      for (int ii = 0; ii < QC; ++ii)
+        if (ii < ni)
 #pragma unroll
-          for (int j = 0; j < NV; ++j) acc[ii * NV + j] = fma(qv, v[j], acc[ii * NV + j]);
-        }
-      }
+          for (int j = 0; j < NV; ++j) acc[ii * NV + j] = fma(qv[ii], v[j], acc[ii * NV + j]);
     }
   }
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-#pragma unroll
-  for (int p = 0; p < NP; ++p) {
-    const double v = wave_sum(acc[p]);
-    if (lane == 0) sh[wave * NP + p] = v;
-  }
+  // the wave butterflies, then the four waves left to right (block_sum's tree)
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, slot = sum_slot(lane);
+  const double ws = wave_sum_lanes<NP, 32>(acc);
+  if (slot < NP) sh[wave * NP + slot] = ws;
   __syncthreads();
   for (int p = threadIdx.x; p < NP; p += blockDim.x) {
     const int ii = p / NV, j = p % NV;
@@ -296,25 +374,45 @@ __global__ void __launch_bounds__(kNT) k_ca_reduce_slots(const double* part, int
   if (threadIdx.x == 0) out[blockIdx.x] = v;
 }
 
-// V_j -= sum_i R'(i,j) Q_i for j = 1..nv (columns of V), i = 0..c1-1 in
+// V_j -= sum_i R'(i,j) Q_i for j = 1..NV (columns of V), i = 0..c1-1 in
 // order, as fma(-R'(i,j), Q_i, .) (calc_gemm with the negated R',
-// vec.f90:403-440); R' is c1 x (nv+1), ld c1, column 0 unused
-__global__ void __launch_bounds__(kNT) k_ca_bupd(int n, const double* Q, long ldq, int c1, double* V, long ldv,
-                                                 int nv, const double* Rp) {
+// vec.f90:403-440); R' is c1 x (NV+1), ld c1, column 0 unused.  Bound by
+// reading Q and V once and writing V: the NV columns of a row stay in
+// registers, the Q columns are loaded kBU at a time before their products
+// (one load in flight per row left it at 1.7 TB/s), and -R' lies in LDS where
+// a wavefront reads one entry as a broadcast.  n = 2^21, NV = 8, c1 = 17
+// (mean over 9, 17, 25): 345 us before, 98 us now.
+constexpr int kBU = 4;
+template <int NV>
+__global__ void __launch_bounds__(kNT) k_ca_bupd(int n, const double* __restrict__ Q, long ldq, int c1, double* V,
+                                                 long ldv, const double* __restrict__ Rp) {
+  extern __shared__ double nr[];  // -R'(i, j) at i * NV + j - 1
+  for (int e = threadIdx.x; e < c1 * NV; e += blockDim.x) {
+    const int i = e / NV, j = e - i * NV + 1;
+    nr[e] = -Rp[i + (long)c1 * j];
+  }
+  __syncthreads();
   for (long q = (long)blockIdx.x * blockDim.x + threadIdx.x; q < n; q += (long)gridDim.x * blockDim.x) {
-    double w[kMaxCols];
+    double w[NV];
 #pragma unroll
-    for (int j = 0; j < kMaxCols; ++j)
-      if (j < nv) w[j] = V[(long)(j + 1) * ldv + q];
-    for (int i = 0; i < c1; ++i) {
+    for (int j = 0; j < NV; ++j) w[j] = V[(long)(j + 1) * ldv + q];
+    int i = 0;
+    for (; i + kBU <= c1; i += kBU) {
+      double qv[kBU];
+#pragma unroll
+      for (int u = 0; u < kBU; ++u) qv[u] = Q[(long)(i + u) * ldq + q];
+#pragma unroll
+      for (int u = 0; u < kBU; ++u)
+#pragma unroll
+        for (int j = 0; j < NV; ++j) w[j] = fma(nr[(i + u) * NV + j], qv[u], w[j]);
+    }
+    for (; i < c1; ++i) {
       const double qv = Q[(long)i * ldq + q];
 #pragma unroll
-      for (int j = 0; j < kMaxCols; ++j)
-        if (j < nv) w[j] = fma(-Rp[i + (long)c1 * (j + 1)], qv, w[j]);
+      for (int j = 0; j < NV; ++j) w[j] = fma(nr[i * NV + j], qv, w[j]);
     }
 #pragma unroll
-    for (int j = 0; j < kMaxCols; ++j)
-      if (j < nv) V[(long)(j + 1) * ldv + q] = w[j];
+    for (int j = 0; j < NV; ++j) V[(long)(j + 1) * ldv + q] = w[j];
   }
 }
 
@@ -352,6 +450,55 @@ inline int tsqr_waves(int n) {
   return np < kTsqrWaves ? (np > 0 ? np : 1) : kTsqrWaves;
 }
 
+// Columns I .. NC - 1 of a panel: column I's reflector, applied to the columns
+// right of it and to row I of R (held by lane I).
+template <int NC, int I>
+__device__ __forceinline__ void tsqr_columns(double (&P)[NC], double (&Rrow)[NC], int lane) {
+  if constexpr (I < NC) {
+    constexpr int N = NC - I, N0 = N < 8 ? N : 8, N1 = N - N0;
+    const double x = P[I];
+    double d[N];
+    {
+      double d0[N0];
+#pragma unroll
+      for (int k = 0; k < N0; ++k) d0[k] = x * P[I + k];
+      wave_sum_n<N0>(d0);
+#pragma unroll
+      for (int k = 0; k < N0; ++k) d[k] = d0[k];
+    }
+    if constexpr (N1 > 0) {
+      double d1[N1];
+#pragma unroll
+      for (int k = 0; k < N1; ++k) d1[k] = x * P[I + N0 + k];
+      wave_sum_n<N1>(d1);
+#pragma unroll
+      for (int k = 0; k < N1; ++k) d[N0 + k] = d1[k];
+    }
+    const double alpha = read_lane(Rrow[I], I);
+    const double s2 = d[0];
+    const double nrm = sqrt(fma(alpha, alpha, s2));
+    const double y1 = alpha > 0.0 ? alpha + nrm : alpha - nrm;
+    double den = fma(y1, y1, s2);
+    if (den == 0.0) den = 1.0 - 300;
+    const double t1 = 2.0 / den;
+    const double na = fma(-(t1 * y1), fma(y1, alpha, s2), alpha);
+#pragma unroll
+    for (int k = I + 1; k < NC; ++k) {
+      const double rik = read_lane(Rrow[k], I);
+      const double tk = t1 * fma(y1, rik, d[k - I]);
+      P[k] = fma(-x, tk, P[k]);
+      const double nr = fma(-y1, tk, rik);
+      if (lane == I) Rrow[k] = nr;
+    }
+    if (lane == I) Rrow[I] = na;
+    tsqr_columns<NC, I + 1>(P, Rrow, lane);
+  }
+}
+
+// Bound by the dependent chain of a panel's columns (a wavefront sum, a square
+// root and a division each) on one wavefront per SIMD.  n = 2^21, NC = 8: 201
+// us with one butterfly per sum, 104 us with shared steps and the sums,
+// R entries and reflector scalars in scalar registers.
 template <int NC>
 __global__ void __launch_bounds__(kNT) k_tsqr(int n, const double* V, long ldv, int W, double* Rout) {
   const int lane = threadIdx.x & 63;
@@ -361,40 +508,17 @@ __global__ void __launch_bounds__(kNT) k_tsqr(int n, const double* V, long ldv, 
   double Rrow[NC];
 #pragma unroll
   for (int c = 0; c < NC; ++c) Rrow[c] = 0.0;
+  double Pn[NC];  // the next panel, loaded while this one is folded in
+#pragma unroll
+  for (int c = 0; c < NC; ++c) Pn[c] = (long)w * 64 + lane < n ? V[(long)c * ldv + (long)w * 64 + lane] : 0.0;
   for (int p = w; p < np; p += W) {
-    const long row = (long)p * 64 + lane;
     double P[NC];
 #pragma unroll
-    for (int c = 0; c < NC; ++c) P[c] = row < n ? V[(long)c * ldv + row] : 0.0;
+    for (int c = 0; c < NC; ++c) P[c] = Pn[c];
+    const long row = (long)(p + W) * 64 + lane;
 #pragma unroll
-    for (int i = 0; i < NC; ++i) {
-      const double x = P[i];
-      double d[NC];
-#pragma unroll
-      for (int k = i; k < NC; ++k) d[k] = x * P[k];
-      // the xor butterfly (offsets 32..1) in registers
-#define PARCEL_XSTEP(O) \
-  for (int k = i; k < NC; ++k) d[k] += xor_lane<O>(d[k]);
-      PARCEL_XSTEP(32) PARCEL_XSTEP(16) PARCEL_XSTEP(8) PARCEL_XSTEP(4) PARCEL_XSTEP(2) PARCEL_XSTEP(1)
-#undef PARCEL_XSTEP
-      const double alpha = __shfl(Rrow[i], i, 64);
-      const double s2 = d[i];
-      const double nrm = sqrt(fma(alpha, alpha, s2));
-      const double y1 = alpha > 0.0 ? alpha + nrm : alpha - nrm;
-      double den = fma(y1, y1, s2);
-      if (den == 0.0) den = 1.0 - 300;
-      const double t1 = 2.0 / den;
-      const double na = fma(-(t1 * y1), fma(y1, alpha, s2), alpha);
-#pragma unroll
-      for (int k = i + 1; k < NC; ++k) {
-        const double rik = __shfl(Rrow[k], i, 64);
-        const double tk = t1 * fma(y1, rik, d[k]);
-        P[k] = fma(-x, tk, P[k]);
-        const double nr = fma(-y1, tk, rik);
-        if (lane == i) Rrow[k] = nr;
-      }
-      if (lane == i) Rrow[i] = na;
-    }
+    for (int c = 0; c < NC; ++c) Pn[c] = row < n ? V[(long)c * ldv + row] : 0.0;
+    tsqr_columns<NC, 0>(P, Rrow, lane);
   }
   if (lane < NC) {
 #pragma unroll
@@ -472,6 +596,19 @@ void bdots(int nv, dim3 grid, hipStream_t st, int n, const double* Q, long ldq, 
     PARCEL_BD(10) PARCEL_BD(11) PARCEL_BD(12) PARCEL_BD(13) PARCEL_BD(14) PARCEL_BD(15) PARCEL_BD(16)
 #undef PARCEL_BD
     default: throw hip_error("CA-GMRES: s + 1 must be in 2..16", PARCEL_HIP_ERR_ARG);
+  }
+}
+
+void bupd(int nv, dim3 grid, hipStream_t st, int n, const double* Q, long ldq, int c1, double* V, long ldv,
+          const double* Rp) {
+  const size_t shm = sizeof(double) * (size_t)c1 * nv;  // at most 128 * 15 entries
+  switch (nv) {
+#define PARCEL_BU(C) \
+  case C: hipLaunchKernelGGL(k_ca_bupd<C>, grid, dim3(kNT), shm, st, n, Q, ldq, c1, V, ldv, Rp); break;
+    PARCEL_BU(1) PARCEL_BU(2) PARCEL_BU(3) PARCEL_BU(4) PARCEL_BU(5) PARCEL_BU(6) PARCEL_BU(7) PARCEL_BU(8)
+    PARCEL_BU(9) PARCEL_BU(10) PARCEL_BU(11) PARCEL_BU(12) PARCEL_BU(13) PARCEL_BU(14) PARCEL_BU(15)
+#undef PARCEL_BU
+    default: throw hip_error("CA-GMRES: s must be in 1..15", PARCEL_HIP_ERR_ARG);
   }
 }
 
@@ -770,10 +907,9 @@ int cagmres_solve(Plan& P, double* x, const double* b, int itrmax, double rtol, 
       } else {
         // block CGS: R' = Q(:,1:c1)^T V, V(:,2:s+1) -= Q(:,1:c1) R'(:,2:s+1)
         const int c1 = s * (k - 1) + 1;
-        bdots(nc, dim3(nb, (c1 + 3) / 4), st, n, Q, ldv, c1, V, ldv, gp);
+        bdots(nc, dim3(nb, (c1 + bdots_cols(nc) - 1) / bdots_cols(nc)), st, n, Q, ldv, c1, V, ldv, gp);
         hipLaunchKernelGGL(k_ca_reduce_slots, dim3(c1 * nc), block, 0, st, (const double*)gp, nb, dRp);
-        hipLaunchKernelGGL(k_ca_bupd, grid, block, 0, st, n, (const double*)Q, ldv, c1, V, ldv, s,
-                           (const double*)dRp);
+        bupd(s, grid, st, n, Q, ldv, c1, V, ldv, dRp);
         launches += 3;
         PARCEL_HIP_CHECK(hipMemcpyAsync(hRp, dRp, sizeof(double) * (size_t)c1 * nc, hipMemcpyDeviceToHost, st));
         std::vector<double> Rk((size_t)s * s, 0.0);
