@@ -22,6 +22,7 @@
 #include <vector>
 
 #include "dense.hpp"
+#include "house.hpp"
 #include "kernels.hpp"
 
 namespace parcel {
@@ -443,7 +444,7 @@ __global__ void __launch_bounds__(kNT) k_ca_vrinv(int n, const double* V, long l
 // by Householder QR of [R; P], House_local_Ronly_omp's reflector
 // v = [y1; P(:,i)] on the stacked matrix: the 64-lane sums are xor
 // butterflies, the R entries are broadcast from their row's lane.  The W
-// factors go to Rout (NC x NC each, column-major) for the host's second level.
+// factors go to Rout (stacked, row by row) for the host's second level.
 constexpr int kTsqrWaves = 1024;
 inline int tsqr_waves(int n) {
   const int np = (n + 63) / 64;
@@ -522,7 +523,7 @@ __global__ void __launch_bounds__(kNT) k_tsqr(int n, const double* V, long ldv, 
   }
   if (lane < NC) {
 #pragma unroll
-    for (int c = 0; c < NC; ++c) Rout[(long)w * NC * NC + lane + c * NC] = (c >= lane) ? Rrow[c] : 0.0;
+    for (int c = 0; c < NC; ++c) Rout[((long)w * NC + lane) * NC + c] = (c >= lane) ? Rrow[c] : 0.0;
   }
 }
 
@@ -669,11 +670,12 @@ void tsqr_r(int n, int nc, const double* V, long ldv, double* dT, double* hT, do
   PARCEL_HIP_CHECK(hipMemcpyAsync(hT, dT, sizeof(double) * (size_t)W * nc * nc, hipMemcpyDeviceToHost, st));
   PARCEL_HIP_CHECK(hipStreamSynchronize(st));
   const int mrows = W * nc;
-  std::vector<double> S((size_t)mrows * nc);
-  for (int w = 0; w < W; ++w)
-    for (int j = 0; j < nc; ++j)
-      for (int i = 0; i < nc; ++i) S[(size_t)w * nc + i + (size_t)j * mrows] = hT[(size_t)w * nc * nc + i + (size_t)j * nc];
-  dense::house_r(mrows, nc, S.data(), mrows, R);
+  if (!house_r_rows(mrows, nc, hT, R)) {
+    std::vector<double> S((size_t)mrows * nc);
+    for (int i = 0; i < mrows; ++i)
+      for (int j = 0; j < nc; ++j) S[i + (size_t)j * mrows] = hT[(size_t)i * nc + j];
+    dense::house_r(mrows, nc, S.data(), mrows, R);
+  }
   for (int j = 0; j < nc; ++j)
     if (R[j + (size_t)j * nc] < 0.0)
       for (int i = j; i < nc; ++i) R[j + (size_t)i * nc] = -R[j + (size_t)i * nc];
