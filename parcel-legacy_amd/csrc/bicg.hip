@@ -34,7 +34,7 @@ __global__ void __launch_bounds__(kNT) k_spmv_dots(int n, SellArgs A, const doub
                                                    double* __restrict__ y, const double* __restrict__ u,
                                                    double* part, int slot0, int slot1, const int* skip) {
   if (*skip) return;
-  __shared__ double sh[kWaves];
+  __shared__ double sh[kWaves * ND];
   const int nb = gridDim.x;
   const long ntiles = ((long)n + kNT - 1) / kNT;
   double acc[2] = {0.0, 0.0};
@@ -67,48 +67,42 @@ __global__ void __launch_bounds__(kNT) k_bi_init(const double* part, int nb, BiS
   }
 }
 
-// top of iteration: history, c2, alpha (pbicg.f90:470-500)
-__global__ void __launch_bounds__(kNT) k_bi_alpha(const double* part, int nb, BiState* st, double* hist,
-                                                  int hist_cap) {
+// The scalars of an iteration are reduced by the kernel that uses them, in
+// every workgroup alike (reduce_part's tree); workgroup 0 writes them down.
+// A kernel of their own cost 3.4 us and a launch gap each, three times an
+// iteration: 75 x 61 x 43 (D-ILU) took 100 us an iteration with them, 87 without.
+
+// top of iteration: history, c2, alpha (pbicg.f90:470-500); e = r - alpha q
+__global__ void __launch_bounds__(kNT) k_bi_e(int n, const double* __restrict__ r, const double* __restrict__ q,
+                                              double* __restrict__ e, const double* part, int nb, BiState* st,
+                                              double* hist, int hist_cap) {
   if (st->done) return;
   __shared__ double sh[kWaves];
   const double c2 = reduce_part(part + BP_C2 * kNBMax, nb, sh);
-  if (threadIdx.x == 0) {
+  const double alpha = st->c1 / c2;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
     const int itr = st->itr + 1;
     if (itr - 1 < hist_cap) hist[itr - 1] = st->rnorm / st->bnorm;
     st->itr = itr;
     st->c2 = c2;
-    st->alpha = st->c1 / c2;
+    st->alpha = alpha;
   }
-}
-
-// e = r - alpha q
-__global__ void __launch_bounds__(kNT) k_bi_e(int n, const double* __restrict__ r, const double* __restrict__ q,
-                                              double* __restrict__ e, const BiState* st) {
-  if (st->done) return;
-  const double alpha = st->alpha;
   for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x)
     e[i] = fma(-alpha, q[i], r[i]);
 }
 
-// c3 = <e,v> / <v,v>
-__global__ void __launch_bounds__(kNT) k_bi_c3(const double* part, int nb, BiState* st) {
-  if (st->done) return;
-  __shared__ double sh[kWaves];
-  const double ev = reduce_part(part + BP_EV * kNBMax, nb, sh);
-  const double vv = reduce_part(part + BP_VV * kNBMax, nb, sh);
-  if (threadIdx.x == 0) st->c3 = ev / vv;
-}
-
-// x += alpha pp + c3 pe ; r = e - c3 v ; partials <r,r0>, <r,r>  (BiCG_axpy3_dot)
+// c3 = <e,v> / <v,v>; x += alpha pp + c3 pe ; r = e - c3 v ; partials <r,r0>, <r,r>  (BiCG_axpy3_dot)
 __global__ void __launch_bounds__(kNT) k_bi_update(int n, double* __restrict__ x, const double* __restrict__ pp,
                                                    const double* __restrict__ pe, double* __restrict__ r,
                                                    const double* __restrict__ e, const double* __restrict__ v,
-                                                   const double* __restrict__ r0, double* part, const BiState* st) {
+                                                   const double* __restrict__ r0, double* part, BiState* st) {
   if (st->done) return;
-  __shared__ double sh[kWaves];
-  const double alpha = st->alpha, c3 = st->c3;
+  __shared__ double sh2[kWaves * 2];
   const int nb = gridDim.x;
+  double ev, vv;
+  reduce_part2(part + BP_EV * kNBMax, part + BP_VV * kNBMax, nb, sh2, ev, vv);
+  const double alpha = st->alpha, c3 = ev / vv;
+  if (blockIdx.x == 0 && threadIdx.x == 0) st->c3 = c3;
   const long ntiles = ((long)n + kNT - 1) / kNT;
   double acc[2] = {0.0, 0.0};
   for (long k = blockIdx.x; k < ntiles; k += nb) {
@@ -122,37 +116,36 @@ __global__ void __launch_bounds__(kNT) k_bi_update(int n, double* __restrict__ x
     }
   }
   const int slots[2] = {BP_C1, BP_RR};
-  store_partials<2>(part, slots, acc, sh);
+  store_partials<2>(part, slots, acc, sh2);
 }
 
-// exit test and beta (pbicg.f90:590-625)
-__global__ void __launch_bounds__(kNT) k_bi_beta(const double* part, int nb, BiState* st, int itrmax,
-                                                 double rtol) {
+// exit test and beta (pbicg.f90:590-625); p = r - beta c3 q + beta p.  (A
+// workgroup that starts after workgroup 0 has set `done` here returns at once,
+// as it would from its own exit test.)
+__global__ void __launch_bounds__(kNT) k_bi_p(int n, double* __restrict__ p, const double* __restrict__ r,
+                                              const double* __restrict__ q, const double* part, int nb, BiState* st,
+                                              int itrmax, double rtol) {
   if (st->done) return;
-  __shared__ double sh[kWaves];
-  const double c1 = reduce_part(part + BP_C1 * kNBMax, nb, sh);
-  const double rr = reduce_part(part + BP_RR * kNBMax, nb, sh);
-  if (threadIdx.x == 0) {
-    const double rnorm = sqrt(rr);
+  __shared__ double sh2[kWaves * 2];
+  double c1, rr;
+  reduce_part2(part + BP_C1 * kNBMax, part + BP_RR * kNBMax, nb, sh2, c1, rr);
+  const double rnorm = sqrt(rr), c3 = st->c3;
+  const int itr = st->itr;
+  const bool last = rnorm / st->bnorm < rtol || itr >= itrmax;
+  const double beta = c1 / (c3 * st->c2);
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
     st->rnorm = rnorm;
     st->c1 = c1;
-    const int itr = st->itr;
-    if (rnorm / st->bnorm < rtol || itr >= itrmax) {
+    if (last) {
       st->done = 1;
-      st->niter = itr;                    // min(itrmax, itr)
+      st->niter = itr;                     // min(itrmax, itr)
       st->iret = (itrmax <= itr) ? 1 : 0;  // pbicg.f90:672-676
     } else {
-      st->beta = c1 / (st->c3 * st->c2);
+      st->beta = beta;
     }
   }
-}
-
-// p = r - beta c3 q + beta p
-__global__ void __launch_bounds__(kNT) k_bi_p(int n, double* __restrict__ p, const double* __restrict__ r,
-                                              const double* __restrict__ q, const BiState* st) {
-  if (st->done) return;
-  const double beta = st->beta;
-  const double bc = -(beta * st->c3);
+  if (last) return;
+  const double bc = -(beta * c3);
   for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x)
     p[i] = fma(beta, p[i], fma(bc, q[i], r[i]));
 }
@@ -208,17 +201,16 @@ int bicg_solve(Plan& P, double* x, const double* b, int itrmax, double rtol, dou
       precon_apply(P, p, pp, nullptr, done);
       hipLaunchKernelGGL(k_spmv_dots<1>, grid, block, 0, st, n, A, (const double*)pp, q, (const double*)r0, part,
                          (int)BP_C2, 0, done);
-      hipLaunchKernelGGL(k_bi_alpha, dim3(1), block, 0, st, (const double*)part, nb, S, P.hist.p, P.hist_cap);
-      hipLaunchKernelGGL(k_bi_e, grid, block, 0, st, n, (const double*)r, (const double*)q, e, (const BiState*)S);
+      hipLaunchKernelGGL(k_bi_e, grid, block, 0, st, n, (const double*)r, (const double*)q, e, (const double*)part, nb,
+                         S, P.hist.p, P.hist_cap);
       precon_apply(P, e, pe, nullptr, done);
       hipLaunchKernelGGL(k_spmv_dots<2>, grid, block, 0, st, n, A, (const double*)pe, v, (const double*)e, part,
                          (int)BP_EV, (int)BP_VV, done);
-      hipLaunchKernelGGL(k_bi_c3, dim3(1), block, 0, st, (const double*)part, nb, S);
       hipLaunchKernelGGL(k_bi_update, grid, block, 0, st, n, x, (const double*)pp, (const double*)pe, r,
-                         (const double*)e, (const double*)v, (const double*)r0, part, (const BiState*)S);
-      hipLaunchKernelGGL(k_bi_beta, dim3(1), block, 0, st, (const double*)part, nb, S, itrmax, rtol);
-      hipLaunchKernelGGL(k_bi_p, grid, block, 0, st, n, p, (const double*)r, (const double*)q, (const BiState*)S);
-      launches += 10;
+                         (const double*)e, (const double*)v, (const double*)r0, part, S);
+      hipLaunchKernelGGL(k_bi_p, grid, block, 0, st, n, p, (const double*)r, (const double*)q, (const double*)part, nb,
+                         S, itrmax, rtol);
+      launches += 7;
     }
     PARCEL_HIP_CHECK(hipGetLastError());
     enq += k;

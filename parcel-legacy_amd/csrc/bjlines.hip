@@ -186,17 +186,17 @@ __host__ __device__ __forceinline__ dd dd_div_one(dd z) {
 }
 
 // One sweep of a block.  NR: steps the factor operands are loaded ahead.
-template <bool FWD, int MODE, bool FUSED, bool PL, bool MULTI, int NV, int NR>
-__device__ __forceinline__ void line_sweep(const LineArgs& A, const LineBlock bk, int w, int W,
+// alphaf: the fused update's alpha, asked for once the first loads are out.
+template <bool FWD, int MODE, bool FUSED, bool PL, bool MULTI, int NV, int NR, class AF>
+__device__ __forceinline__ void line_sweep(const LineArgs& A, const LineBlock bk, const LineWave wv, int w, int W,
                                            const typename Num<NV>::Vec in, const typename Num<NV>::Vec out,
-                                           const typename Num<NV>::Vec q, double alpha, typename Num<NV>::L* lds) {
+                                           const typename Num<NV>::Vec q, AF alphaf, typename Num<NV>::L* lds) {
   using N = Num<NV>;
   using V = typename N::V;
   constexpr bool kScale = !(FWD && MODE == BJ_ILU0);
   constexpr int NE = (PL ? 1 : 0) + (kScale ? 1 : 0);
   const int nx = A.nx;
   const int lane = threadIdx.x & 63;
-  const LineWave wv = (FWD ? A.fw : A.bw)[(long)blockIdx.x * W + w];
   const int dir = FWD ? 0 : 1;
   const int ng = FWD ? bk.ngf : bk.ngb;
   constexpr int sg = FWD ? 1 : -1;
@@ -263,6 +263,7 @@ __device__ __forceinline__ void line_sweep(const LineArgs& A, const LineBlock bk
   auto chunk_off = [&](int ri, int ci, int k) -> int {
     return (unsigned)(ci - 64 * k) < lenk[k] ? (int)((unsigned)ri + k * kst) : kOOB;
   };
+  double alpha = 0.0;
   V va[2][8], vb[FUSED ? 2 : 1][FUSED ? 8 : 1];
   int mo[FUSED ? 2 : 1][FUSED ? 8 : 1];
   auto stage_load = [&](auto pc, int ri, int ci) {
@@ -408,6 +409,7 @@ __device__ __forceinline__ void line_sweep(const LineArgs& A, const LineBlock bk
   using P1 = std::integral_constant<int, 1>;
   stage_load(P0{}, ri - sg * 64, ci - 64);
   stage_load(P1{}, ri, ci);
+  if constexpr (FUSED) alpha = alphaf();
   stage_fill(P0{}, sb);             // slot of group -2 == group 1
   stage_fill(P1{}, next_slot(sb));  // slot of group -1 == group 2
   ri += sg * 64;
@@ -444,18 +446,19 @@ __device__ __forceinline__ typename Num<NV>::Vec line_vec(const double* h, const
 template <int MODE, int NTH, bool PL, bool FUSED>
 __global__ void __launch_bounds__(NTH) k_bj_lines(LineArgs A, const double* rin, double* s, CGFuse fuse,
                                                   const int* skip) {
-  if (skip && *skip) return;
   extern __shared__ double lds_lines[];
   __shared__ double sh[kWaves];
   constexpr bool MULTI = NTH > 64;
   constexpr int NR = NTH > 256 ? 8 : 16;
   const int W = MULTI ? (int)(blockDim.x >> 6) : 1;
   const int w = MULTI ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
-  double alpha = 0.0;
-  if constexpr (FUSED) {
-    const int d = fuse.st->done_at;
-    if (d != 0 && d <= fuse.it) return;
-    CGSlot* sl = &fuse.st->slot[fuse.it & 1];
+  // the state and the tables are read together
+  const int done = FUSED ? fuse.st->done_at : skip ? *skip : 0;
+  const LineBlock bk = A.blk[blockIdx.x];
+  const LineWave wf = A.fw[(long)blockIdx.x * W + w], wb = A.bw[(long)blockIdx.x * W + w];
+  if (done != 0 && (!FUSED || done <= fuse.it)) return;
+  auto alphaf = [&]() -> double {
+    CGSlot* slot = &fuse.st->slot[fuse.it & 1];
     for (int vw = w; vw < kWaves; vw += W) {
       double a = 0.0;
       for (int j = vw * 64 + (threadIdx.x & 63); j < fuse.nb_prod; j += kNT) a = a + fuse.part_gamma[j];
@@ -465,34 +468,38 @@ __global__ void __launch_bounds__(NTH) k_bj_lines(LineArgs A, const double* rin,
     __syncthreads();
     double gamma = sh[0];
     for (int k = 1; k < kWaves; ++k) gamma = gamma + sh[k];
-    alpha = sl->rho0 / gamma;
-    if (blockIdx.x == 0 && threadIdx.x == 0) sl->alpha = alpha;
-  }
-  const LineBlock bk = A.blk[blockIdx.x];
+    const double alpha = slot->rho0 / gamma;
+    if (blockIdx.x == 0 && threadIdx.x == 0) slot->alpha = alpha;
+    return alpha;
+  };
+  auto none = []() -> double { return 0.0; };
   using Vec = Num<1>::Vec;
   const Vec vs = line_vec<1>(s, nullptr, bk);
   const Vec vr = line_vec<1>(FUSED ? fuse.r : rin, nullptr, bk);
   const Vec vq = line_vec<1>(FUSED ? fuse.q : rin, nullptr, bk);
-  line_sweep<true, MODE, FUSED, PL, MULTI, 1, NR>(A, bk, w, W, vr, vs, vq, alpha, lds_lines);
+  line_sweep<true, MODE, FUSED, PL, MULTI, 1, NR>(A, bk, wf, w, W, vr, vs, vq, alphaf, lds_lines);
   __syncthreads();  // forward values in memory before other threads' backward rows read them
-  line_sweep<false, MODE, false, PL, MULTI, 1, NR>(A, bk, w, W, vs, vs, vs, 0.0, lds_lines);
+  line_sweep<false, MODE, false, PL, MULTI, 1, NR>(A, bk, wb, w, W, vs, vs, vs, none, lds_lines);
 }
 
 template <int MODE, int NTH, bool PL>
 __global__ void __launch_bounds__(NTH) k_bj_lines_dd(LineArgs A, const double* rh, const double* rl, double* sh,
                                                      double* sl, const int* skip) {
-  if (skip && *skip) return;
   extern __shared__ double lds_lines[];
   constexpr bool MULTI = NTH > 64;
   const int W = MULTI ? (int)(blockDim.x >> 6) : 1;
   const int w = MULTI ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
+  const int done = skip ? *skip : 0;
   const LineBlock bk = A.blk[blockIdx.x];
+  const LineWave wf = A.fw[(long)blockIdx.x * W + w], wb = A.bw[(long)blockIdx.x * W + w];
+  if (done) return;
   using Vec = Num<2>::Vec;
   const Vec vs = line_vec<2>(sh, sl, bk), vr = line_vec<2>(rh, rl, bk);
   dd16* lds = reinterpret_cast<dd16*>(lds_lines);
-  line_sweep<true, MODE, false, PL, MULTI, 2, 4>(A, bk, w, W, vr, vs, vs, 0.0, lds);
+  auto none = []() -> double { return 0.0; };
+  line_sweep<true, MODE, false, PL, MULTI, 2, 4>(A, bk, wf, w, W, vr, vs, vs, none, lds);
   __syncthreads();  // forward values in memory before other threads' backward rows read them
-  line_sweep<false, MODE, false, PL, MULTI, 2, 4>(A, bk, w, W, vs, vs, vs, 0.0, lds);
+  line_sweep<false, MODE, false, PL, MULTI, 2, 4>(A, bk, wb, w, W, vs, vs, vs, none, lds);
 }
 
 size_t line_lds_bytes(int W, int parts) { return sizeof(double) * (size_t)parts * (64 * (size_t)W + 1) * kLL; }

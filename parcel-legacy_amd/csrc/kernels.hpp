@@ -72,15 +72,54 @@ __device__ __forceinline__ double reduce_part(const double* part, int nb, double
   return block_sum(a, sh);
 }
 
+// N workgroup sums at once, each equal to block_sum's (butterfly per wave,
+// then the wave totals left to right); sh must hold kWaves*N doubles.
+template <int N>
+__device__ __forceinline__ void block_sum_n(double (&v)[N], double* sh) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+#pragma unroll
+  for (int d = 0; d < N; ++d) v[d] = wave_sum(v[d]);
+  __syncthreads();
+  if (lane == 0) {
+#pragma unroll
+    for (int d = 0; d < N; ++d) sh[w * N + d] = v[d];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int d = 0; d < N; ++d) {
+    double t = sh[d];
+#pragma unroll
+    for (int k = 1; k < kWaves; ++k) t = t + sh[k * N + d];
+    v[d] = t;
+  }
+}
+
+// Two of reduce_part's reductions at once (the same trees): both sets of
+// partials in flight together, one pair of barriers.  sh: 2 kWaves doubles.
+__device__ __forceinline__ void reduce_part2(const double* pa, const double* pb, int nb, double* sh, double& ra,
+                                             double& rb) {
+  double v[2] = {0.0, 0.0};
+  for (int j = threadIdx.x; j < nb; j += kNT) {
+    v[0] = v[0] + pa[j];
+    v[1] = v[1] + pb[j];
+  }
+  block_sum_n<2>(v, sh);
+  ra = v[0];
+  rb = v[1];
+}
 
 // Partials of up to three dot products over the tiled layout, written to
-// part[slot0], part[slot1], part[slot2] (each kNBMax doubles apart).
+// part[slot0], part[slot1], part[slot2] (each kNBMax doubles apart); sh: kWaves
+// doubles per product.
 template <int ND>
 __device__ __forceinline__ void store_partials(double* part, const int* slots, const double* acc, double* sh) {
+  double v[ND];
 #pragma unroll
-  for (int d = 0; d < ND; ++d) {
-    const double v = block_sum(acc[d], sh);
-    if (threadIdx.x == 0) part[slots[d] * kNBMax + blockIdx.x] = v;
+  for (int d = 0; d < ND; ++d) v[d] = acc[d];
+  block_sum_n<ND>(v, sh);
+  if (threadIdx.x == 0) {
+#pragma unroll
+    for (int d = 0; d < ND; ++d) part[slots[d] * kNBMax + blockIdx.x] = v[d];
   }
 }
 
