@@ -33,10 +33,12 @@
 // CU (256 planes of 256 x 256) HBM bounds it.
 // Measured, one apply, against the kernels before (a line form for whole lines
 // and planes with addresses selected per lane; level-scheduled sweeps for the
-// others): 64 blocks of two 128 x 128 planes ILU(0) 157 -> 91 us; 256 planes of
+// others): 64 blocks of two 128 x 128 planes ILU(0) 157 -> 92 us; 256 planes of
 // 256 x 256 with the fused update 374 -> 366 us in the solve; 80 blocks of two
-// 160 x 160 planes D-ILU 813 -> 245 us; 256 blocks of 10 1/4 lines of 75 cells
-// D-ILU 136 -> 24 us.
+// 160 x 160 planes D-ILU 813 -> 199 us; 256 blocks of 10 1/4 lines of 75 cells
+// D-ILU 136 -> 23 us.  Double-double, 32 blocks of three 96 x 96 planes ILU(0)
+// (level-scheduled before): 675 -> 350 us, bound by FP64 issue (six wavefronts
+// on four SIMDs).
 #include <algorithm>
 #include <cstdlib>
 #include <type_traits>
@@ -243,7 +245,8 @@ __device__ __forceinline__ void line_sweep(const LineArgs& A, const LineBlock bk
   // Staging: lane 8 j + c moves element c of the 8-row chunk of local line
   // 8 k + j, k = 0..7.  in(g) is the line's chunk (rows aligned to 8) that
   // holds the cell of step 8 g + 15: loaded during group g - 1, put into the
-  // ring after group g and, swept, stored after group g + 2.  For k = 0 and
+  // ring after group g and, swept by the end of group g + 2, stored during
+  // group g + 3.  For k = 0 and
   // the g to load next: ri the byte offset of the element's row, ci 8 times
   // its cell; line 8 k is k (8 nx - 8) rows and -8 k cells away.
   const int sj = lane >> 3, sc = lane & 7;
@@ -266,17 +269,18 @@ __device__ __forceinline__ void line_sweep(const LineArgs& A, const LineBlock bk
   double alpha = 0.0;
   V va[2][8], vb[FUSED ? 2 : 1][FUSED ? 8 : 1];
   int mo[FUSED ? 2 : 1][FUSED ? 8 : 1];
-  auto stage_load = [&](auto pc, int ri, int ci) {
+  auto stage_load_k = [&](auto pc, int ri, int ci, int k) {
     constexpr int p = decltype(pc)::value;
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      const int off = chunk_off(ri, ci, k);
-      va[p][k] = in.load(off);
-      if constexpr (FUSED) {
-        vb[p][k] = q.load(off);
-        mo[p][k] = off;
-      }
+    const int off = chunk_off(ri, ci, k);
+    va[p][k] = in.load(off);
+    if constexpr (FUSED) {
+      vb[p][k] = q.load(off);
+      mo[p][k] = off;
     }
+  };
+  auto stage_load = [&](auto pc, int ri, int ci) {
+#pragma unroll
+    for (int k = 0; k < 8; ++k) stage_load_k(pc, ri, ci, k);
   };
   auto stage_fill = [&](auto pc, int slot) {
     constexpr int p = decltype(pc)::value;
@@ -362,8 +366,6 @@ __device__ __forceinline__ void line_sweep(const LineArgs& A, const LineBlock bk
   auto group = [&](auto pc) {
     constexpr int p = decltype(pc)::value;
     using Q = std::integral_constant<int, 1 - p>;
-    // in(g + 1)
-    stage_load(Q{}, ri, ci);
     wave_lds_sync();
     auto input = [&](int u, V& a, V& h, V& pl) {
       a = N::get(own[s0 + u]);
@@ -378,18 +380,21 @@ __device__ __forceinline__ void line_sweep(const LineArgs& A, const LineBlock bk
     for (int u = 0; u < NI; ++u) hv[u] = pv[u] = N::num(kZero);
 #pragma unroll
     for (int u = 0; u < (NV == 1 ? kLG : 1); ++u) input(u, av[u], hv[u], pv[u]);
+    // the swept chunk in(g - 3), four groups behind ri, out of the slots that
+    // in(g) takes after the steps
+    stage_load(Q{}, ri, ci);
+    V ov[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) ov[k] = N::get(stg[8 * k * kLL + sa]);
+    // a step, the factor operands NR steps ahead and an eighth of the swept
+    // chunk (stores all after the steps: 160^3 on 80 blocks 199 -> 211 us, the
+    // next chunk's loads spread over the steps too: 205 us)
 #pragma unroll
     for (int u = 0; u < kLG; ++u) {
       if (NV == 2 && u + 1 < kLG) input(u + 1, av[(u + 1) % NI], hv[(u + 1) % NI], pv[(u + 1) % NI]);
       own[s0 + u] = N::put(step(u, av[u % NI], hv[u % NI], pv[u % NI], R[(p * kLG + u) % NR]));
       load(u + NR, R[(p * kLG + u) % NR]);
-    }
-    wave_lds_sync();
-    // the swept chunk in(g - 2), three groups behind ri
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      const int off = chunk_off(ri - sg * 3 * 64, ci - 3 * 64, k);
-      out.store(N::get(stg[8 * k * kLL + sb]), off);
+      out.store(ov[u], chunk_off(ri - sg * 4 * 64, ci - 4 * 64, u));
     }
     if (MULTI) lds_barrier();
     else wave_lds_sync();
@@ -426,7 +431,7 @@ __device__ __forceinline__ void line_sweep(const LineArgs& A, const LineBlock bk
   group(P1{});
   for (int g = 2; g < ng; g += 2) {
     group(P0{});
-    group(P1{});
+    if (g + 1 < ng) group(P1{});
   }
 }
 
@@ -586,8 +591,7 @@ bool line_setup_at(Plan& P, const std::vector<BlockSweep>& F, const std::vector<
           e += (nx + v.nl - 1) * v.nl;
           nsteps = std::max(nsteps, v.tw + v.nl - 1 + X);
         }
-      const int g = (nsteps - 1) / kLG + 2;
-      ng[dir] = g + (g & 1);
+      ng[dir] = std::max(2, (nsteps - 1) / kLG + 3);
       if (dir == 1) ents = e;  // both sweeps cut the lines alike: the same number of entries
     }
     blk[b] = LineBlock{blo[b], bhi[b] - blo[b], ng[0], ng[1]};

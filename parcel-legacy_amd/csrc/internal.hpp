@@ -176,7 +176,7 @@ struct LscanBJ {
 // of one step are contiguous.
 struct LineBlock {
   int lo, len;   // the block's rows [lo, lo + len)
-  int ngf, ngb;  // groups of steps of the forward / backward sweep (even)
+  int ngf, ngb;  // groups of steps of the forward / backward sweep (at least 2)
 };
 // One wavefront of a sweep: up to 64 consecutive lines of one plane.  Rows
 // are relative to the block's first row.
