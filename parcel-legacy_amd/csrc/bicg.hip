@@ -193,7 +193,8 @@ int bicg_solve(Plan& P, double* x, const double* b, int itrmax, double rtol, dou
   launches += 2;
   BiState* h = nullptr;
   PARCEL_HIP_CHECK(hipHostMalloc((void**)&h, sizeof(BiState), hipHostMallocDefault));
-  int enq = 0, chunk = 8;
+  ChunkRule rule;
+  int enq = 0, chunk = rule.first();
   const dim3 grid(nb), block(kNT);
   while (enq < itrmax) {
     const int k = std::min(chunk, itrmax - enq);
@@ -217,7 +218,7 @@ int bicg_solve(Plan& P, double* x, const double* b, int itrmax, double rtol, dou
     PARCEL_HIP_CHECK(hipMemcpyAsync(h, S, sizeof(BiState), hipMemcpyDeviceToHost, st));
     PARCEL_HIP_CHECK(hipStreamSynchronize(st));
     if (h->done) break;
-    if (chunk < 64) chunk *= 2;
+    chunk = rule.next(enq, h->rnorm / h->bnorm, rtol);
   }
   PARCEL_HIP_CHECK(hipEventRecord(ev1, st));
   PARCEL_HIP_CHECK(hipMemcpyAsync(h, S, sizeof(BiState), hipMemcpyDeviceToHost, st));

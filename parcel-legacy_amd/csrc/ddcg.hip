@@ -288,7 +288,8 @@ int ddcg_solve(Plan& P, double* xh, double* xl, const double* bh, const double* 
   DDState* h = nullptr;
   PARCEL_HIP_CHECK(hipHostMalloc((void**)&h, sizeof(DDState), hipHostMallocDefault));
   const int* done = &S->done;
-  int it = 1, chunk = 8;
+  ChunkRule rule;
+  int it = 1, chunk = rule.first();
   while (it <= itrmax) {
     const int last = std::min(itrmax, it + chunk - 1);
     for (; it <= last; ++it) {
@@ -311,7 +312,7 @@ int ddcg_solve(Plan& P, double* xh, double* xl, const double* bh, const double* 
     PARCEL_HIP_CHECK(hipMemcpyAsync(h, S, sizeof(DDState), hipMemcpyDeviceToHost, st));
     PARCEL_HIP_CHECK(hipStreamSynchronize(st));
     if (h->done) break;
-    if (chunk < 64) chunk *= 2;
+    chunk = rule.next(it, h->rnorm.hi / h->bnorm.hi, rtol);
   }
   hipLaunchKernelGGL(k_dd_final, grid, block, 0, st, n, xh, xl, (const double*)ph, (const double*)pl,
                      (const DDState*)S);

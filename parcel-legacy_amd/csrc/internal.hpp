@@ -2,6 +2,7 @@
 // translation units of libparcel_hip.so (not part of the public C ABI).
 #pragma once
 
+#include <cmath>
 #include <string>
 #include <vector>
 
@@ -61,6 +62,30 @@ struct PinnedBuf {
   void release() {
     if (p) (void)hipHostFree(p);
     p = nullptr; n = 0;
+  }
+};
+
+// How many iterations a solver enqueues before it looks at the device's state
+// again: 8, 16, 32, then 64, but no more than the iterations that the residual
+// of the last two looks, extended on a logarithmic scale, still needs and two
+// (at least 4).  Launches after convergence return at once but still cost 1 to
+// 2 us each, a look about 15 us; small systems enqueued up to half their
+// iterations for nothing (16^3: 120 for 75).
+struct ChunkRule {
+  int grown = 8, it0 = 0;
+  double l0 = 0.0;
+  int first() const { return grown; }
+  int next(int it, double ratio, double rtol) {
+    if (grown < 64) grown *= 2;
+    int k = grown;
+    const double l = std::log(ratio);
+    if (it0 > 0 && it > it0 && l < l0 && rtol > 0.0 && std::isfinite(l)) {
+      const double need = (l - std::log(rtol)) * (it - it0) / (l0 - l) + 2.0;
+      if (need < k) k = need < 4.0 ? 4 : (int)need;
+    }
+    it0 = it;
+    l0 = l;
+    return k;
   }
 };
 

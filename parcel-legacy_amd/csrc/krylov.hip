@@ -399,7 +399,8 @@ int cg_run(Plan& P, const CGVecs<T>& V, T* x, const T* b, int itrmax, double rto
   CGState* h = P.hstate.p;
   h->done_at = 0;
   int enq = 0;  // K1 launches enqueued
-  int chunk = 8;
+  ChunkRule rule;
+  int chunk = rule.first();
   const bool bj = P.M.kind == PRECON_BJ;
   const bool ras = P.M.kind == PRECON_RAS;
   const bool lscan = std::is_same<T, float>::value && bj && P.M.lscan.on;
@@ -484,7 +485,7 @@ int cg_run(Plan& P, const CGVecs<T>& V, T* x, const T* b, int itrmax, double rto
     PARCEL_HIP_CHECK(hipMemcpyAsync(h, S, sizeof(CGState), hipMemcpyDeviceToHost, st));
     PARCEL_HIP_CHECK(hipStreamSynchronize(st));
     if (h->done_at) break;
-    if (chunk < 64) chunk *= 2;
+    chunk = rule.next(enq, h->slot[enq & 1].rnorm / h->bnorm, rtol);
   }
   PARCEL_HIP_CHECK(hipEventRecord(ev1, st));
   PARCEL_HIP_CHECK(hipMemcpyAsync(h, S, sizeof(CGState), hipMemcpyDeviceToHost, st));
