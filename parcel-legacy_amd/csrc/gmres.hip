@@ -21,6 +21,7 @@
 // multiply/add as written in the reference, with no contraction.
 #include <chrono>
 #include <cmath>
+#include <cstdlib>
 
 #include "kernels.hpp"
 
@@ -40,6 +41,12 @@ struct GmState {
   int done;         // the outer loop has exited
   int niter;
   int iret;
+  int stuck;        // a workgroup gave up waiting in k_gm_column
+  // meetings of k_gm_column's workgroups in one launch: arrivals, and the number
+  // of meetings complete (on lines of their own: the arrivals are atomic adds,
+  // the other word is polled)
+  alignas(128) unsigned arrived;
+  alignas(128) unsigned met;
 };
 
 struct GmArrays {
@@ -51,7 +58,8 @@ struct GmArrays {
   double* h;   // m: CGS coefficients of the current column
 };
 
-__device__ __forceinline__ bool gm_skip(const GmState* st) { return st->done || st->cycle_stop; }
+__device__ __forceinline__ bool gm_halt(const GmState* st) { return st->done || st->stuck; }
+__device__ __forceinline__ bool gm_skip(const GmState* st) { return gm_halt(st) || st->cycle_stop; }
 
 // bnorm = sqrt(<b,b>): partials of the residual kernel, slot 0
 __global__ void __launch_bounds__(kNT) k_gm_init(const double* part, int nb, GmState* st) {
@@ -66,6 +74,9 @@ __global__ void __launch_bounds__(kNT) k_gm_init(const double* part, int nb, GmS
     st->done = 0;
     st->niter = 0;
     st->iret = 0;
+    st->stuck = 0;
+    st->arrived = 0;
+    st->met = 0;
   }
 }
 
@@ -109,8 +120,9 @@ __global__ void __launch_bounds__(kNT) k_gm_scale(int n, const double* __restric
 // w = A pv and the partials of <w, v1> (MGS) or nothing (CGS)
 __global__ void __launch_bounds__(kNT) k_gm_spmv(int n, SellArgs A, const double* __restrict__ pv,
                                                  double* __restrict__ w, const double* __restrict__ v1, double* part,
-                                                 const GmState* st) {
+                                                 GmState* st) {
   if (gm_skip(st)) return;
+  if (blockIdx.x == 0 && threadIdx.x == 0) st->arrived = st->met = 0;  // for the k_gm_column that follows
   __shared__ double sh[kWaves];
   const int nb = gridDim.x;
   const long ntiles = ((long)n + kNT - 1) / kNT;
@@ -215,8 +227,46 @@ __global__ void __launch_bounds__(kNT) k_gm_cgs_update(int n, double* __restrict
   if (threadIdx.x == 0) part[blockIdx.x] = v;
 }
 
-// h_{j+1,j} = sqrt(<w,w>); v_{j+1} = (1/h) w; workgroup 0 applies the Givens
-// rotations to column j and runs the convergence tests (pgmres.f90:385-420)
+// Column j's norm hn into H, the Givens rotations (GivensRotations,
+// src/pcagmres.f90:190-242) and the convergence tests (pgmres.f90:385-420);
+// one thread
+__device__ void gm_givens(GmState* st, const GmArrays& G, int m, int j, int itr, int itrmax, double rtol, double hn,
+                          double* hist, int hist_cap) {
+  double* Hc = G.H + (long)(j - 1) * (m + 1);  // column j
+  Hc[j] = hn;
+  // GivensRotations (src/pcagmres.f90:190-242), column i = j
+  for (int k = 0; k < j - 1; ++k) {
+    const double t1 = Hc[k] * G.c[k] - Hc[k + 1] * G.s[k];
+    const double t2 = Hc[k] * G.s[k] + Hc[k + 1] * G.c[k];
+    Hc[k] = t1;
+    Hc[k + 1] = t2;
+  }
+  double t;
+  if (Hc[j - 1] == 0.0) t = Hc[j] / 1.0 - 300;  // the reference's expression `/1.0d0-300`
+  else t = Hc[j] / Hc[j - 1];
+  const double ci = 1.0 / sqrt(1.0 + t * t);
+  const double si = -ci * t;
+  G.c[j - 1] = ci;
+  G.s[j - 1] = si;
+  const double e1 = ci * G.e[j - 1] - si * G.e[j];
+  const double e2 = si * G.e[j - 1] + ci * G.e[j];
+  G.e[j - 1] = e1;
+  G.e[j] = e2;
+  Hc[j - 1] = ci * Hc[j - 1] - si * Hc[j];
+  Hc[j] = 0.0;
+  const double rnorm = fabs(G.e[j]);
+  st->rnorm = rnorm;
+  st->inner = j;
+  if (itr + j - 1 < hist_cap) hist[itr + j - 1] = rnorm / st->bnorm;
+  if (rnorm / st->bnorm < rtol) {
+    st->converged = 1;
+    st->cycle_stop = 1;
+  } else if (itr + j == itrmax) {
+    st->cycle_stop = 1;
+  }
+}
+
+// h_{j+1,j} = sqrt(<w,w>); v_{j+1} = (1/h) w; workgroup 0 closes column j
 __global__ void __launch_bounds__(kNT) k_gm_norm(int n, const double* __restrict__ w, double* __restrict__ vnext,
                                                  const double* part, int nb_prod, GmState* st, GmArrays G, int m,
                                                  int j, int itr, int itrmax, double rtol, double* hist, int hist_cap) {
@@ -226,45 +276,161 @@ __global__ void __launch_bounds__(kNT) k_gm_norm(int n, const double* __restrict
   const double sc = 1.0 / hn;
   for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x)
     vnext[i] = sc * w[i];
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    double* Hc = G.H + (long)(j - 1) * (m + 1);  // column j
-    Hc[j] = hn;
-    // GivensRotations (src/pcagmres.f90:190-242), column i = j
-    for (int k = 0; k < j - 1; ++k) {
-      const double t1 = Hc[k] * G.c[k] - Hc[k + 1] * G.s[k];
-      const double t2 = Hc[k] * G.s[k] + Hc[k + 1] * G.c[k];
-      Hc[k] = t1;
-      Hc[k + 1] = t2;
+  if (blockIdx.x == 0 && threadIdx.x == 0) gm_givens(st, G, m, j, itr, itrmax, rtol, hn, hist, hist_cap);
+}
+
+// --- MGS of a whole column in one launch ------------------------------------
+//
+// k_gm_mgs moves 32 bytes a row and step: w in and out, v_k, v_{k+1}.  Here w
+// never leaves registers between the SpMV and v_{j+1}: the grid is resident (a
+// cooperative launch of one 1024-thread workgroup per CU), a step reads v_{k+1}
+// alone (v_k is still in registers), and the workgroups meet once a step to
+// exchange the dot's partials.  The loads of the next v are issued before the
+// meeting, so a step takes the longer of 8 n bytes and a meeting.  The sums are
+// k_gm_mgs's: owner o of the tiled layout adds its tiles in order in 256
+// threads (a quarter of a workgroup), partial slot o, reduced by reduce_part's
+// tree in every workgroup.  n = 2^21: 13.2 us a step with k_gm_mgs (and 11.5
+// for the norm), 7.1 here; with release fences in the meetings, which write the
+// L2 back, 28.
+constexpr int kColT = 1024;                  // threads per workgroup
+constexpr int kColQ = kColT / kNT;           // owners worked on at a time
+constexpr unsigned kColSpin = 1u << 20;      // polls before a workgroup gives up (about a second)
+
+// Workgroup barrier that orders LDS accesses only: __syncthreads() would wait
+// for the loads of the next v.
+__device__ __forceinline__ void column_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// Wait for the `count`-th meeting of this launch (one thread).  False when a
+// workgroup was not there within `spin` polls, as when another process holds
+// some of the CUs: every workgroup then leaves (each one's wait is bounded),
+// the rest of the cycle is skipped with x untouched, and the host runs the
+// cycle again with a kernel per step.
+__device__ __forceinline__ bool grid_wait(GmState* st, unsigned count, unsigned spin) {
+  for (unsigned polls = 0; __hip_atomic_load(&st->met, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < count;) {
+    if (++polls > spin || __hip_atomic_load(&st->stuck, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
+      __hip_atomic_store(&st->stuck, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      return false;
     }
-    double t;
-    if (Hc[j - 1] == 0.0) t = Hc[j] / 1.0 - 300;  // the reference's expression `/1.0d0-300`
-    else t = Hc[j] / Hc[j - 1];
-    const double ci = 1.0 / sqrt(1.0 + t * t);
-    const double si = -ci * t;
-    G.c[j - 1] = ci;
-    G.s[j - 1] = si;
-    const double e1 = ci * G.e[j - 1] - si * G.e[j];
-    const double e2 = si * G.e[j - 1] + ci * G.e[j];
-    G.e[j - 1] = e1;
-    G.e[j] = e2;
-    Hc[j - 1] = ci * Hc[j - 1] - si * Hc[j];
-    Hc[j] = 0.0;
-    const double rnorm = fabs(G.e[j]);
-    st->rnorm = rnorm;
-    st->inner = j;
-    if (itr + j - 1 < hist_cap) hist[itr + j - 1] = rnorm / st->bnorm;
-    if (rnorm / st->bnorm < rtol) {
-      st->converged = 1;
-      st->cycle_stop = 1;
-    } else if (itr + j == itrmax) {
-      st->cycle_stop = 1;
-    }
+    __builtin_amdgcn_s_sleep(1);
   }
+  return true;
+}
+
+// Column j: h_kj, k = 1..j, v_{j+1} and the rotations.  part0: the SpMV's
+// partials of <w, v_1>; part: two slots of kNBMax for the later ones.  A
+// workgroup holds OQ * kColQ consecutive owners, OQ per quarter, of RD tiles
+// each (rounds past the vector's end are masked).
+template <int OQ, int RD>
+__global__ void __launch_bounds__(kColT) k_gm_column(int n, const double* __restrict__ w, const double* V, long ldv,
+                                                     double* vnext, const double* part0, double* part, int nb,
+                                                     GmState* st, GmArrays G, int m, int j, int itr, int itrmax,
+                                                     double rtol, double* hist, int hist_cap, unsigned spin) {
+  if (gm_skip(st)) return;  // the state of earlier launches: the same in every workgroup
+  constexpr int E = OQ * RD;
+  __shared__ double sh[OQ][kColT / 64], shr[kWaves];
+  __shared__ int ok;
+  const int q = threadIdx.x / kNT, t = threadIdx.x % kNT, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  // element e = (mo, r): owner o0 + kColQ mo, its tile r
+  const int o0 = blockIdx.x * (OQ * kColQ) + q;
+  const long i0 = (long)o0 * kNT + t;
+  auto index = [&](int e) -> long { return i0 + ((long)(e / RD) * kColQ + (long)(e % RD) * nb) * kNT; };
+  bool in[E];
+#pragma unroll
+  for (int e = 0; e < E; ++e) in[e] = o0 + kColQ * (e / RD) < nb && index(e) < n;
+  double wr[E], v[E], vn[E];
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    wr[e] = in[e] ? w[index(e)] : 0.0;
+    v[e] = in[e] ? V[index(e)] : 0.0;
+  }
+  double hn = 0.0;
+  // v_{k+1} for step k, in flight over the meeting and the reduction
+  auto load_next = [&](int k) {
+    if (k < j) {
+      const double* vk1 = V + (long)k * ldv;
+#pragma unroll
+      for (int e = 0; e < E; ++e) vn[e] = in[e] ? vk1[index(e)] : 0.0;
+    }
+  };
+  load_next(1);
+  for (int k = 1;; ++k) {
+    // h = <w, v_k> (k <= j) or <w, w>: reduce_part's tree in the first 256 threads
+    if (threadIdx.x < kNT) {
+      double a = 0.0;
+      if (k == 1) {
+        for (int p = threadIdx.x; p < nb; p += kNT) a = a + part0[p];
+      } else {
+        const double* pk = part + (k & 1) * kNBMax;
+        double pv[kNBMax / kNT];
+#pragma unroll
+        for (int x = 0; x < kNBMax / kNT; ++x) {
+          const int p = threadIdx.x + x * kNT;
+          pv[x] = p < nb ? __hip_atomic_load(pk + p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0.0;
+        }
+#pragma unroll
+        for (int x = 0; x < kNBMax / kNT; ++x)
+          if ((int)threadIdx.x + x * kNT < nb) a = a + pv[x];
+      }
+      a = wave_sum(a);
+      if (lane == 0) shr[wave] = a;
+    }
+    column_barrier();
+    double h = shr[0];
+#pragma unroll
+    for (int x = 1; x < kWaves; ++x) h = h + shr[x];
+    if (k == j + 1) {
+      hn = sqrt(h);
+      break;
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) G.H[(k - 1) + (long)(j - 1) * (m + 1)] = h;
+    // w -= h v_k; the owners' partials of <w, v_{k+1}>, or <w, w> after the last step
+    double acc[OQ];
+#pragma unroll
+    for (int mo = 0; mo < OQ; ++mo) acc[mo] = 0.0;
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      wr[e] = fma(-h, v[e], wr[e]);
+      v[e] = k < j ? vn[e] : wr[e];
+      if (in[e]) acc[e / RD] = fma(wr[e], v[e], acc[e / RD]);
+    }
+#pragma unroll
+    for (int mo = 0; mo < OQ; ++mo) {
+      const double ws = wave_sum(acc[mo]);
+      if (lane == 0) sh[mo][wave] = ws;
+    }
+    column_barrier();
+    if (t < OQ && o0 + kColQ * t < nb) {
+      double s = sh[t][q * kWaves];
+#pragma unroll
+      for (int x = 1; x < kWaves; ++x) s = s + sh[t][q * kWaves + x];
+      // written through to where every XCD reads it, and there before the
+      // workgroup arrives (a release fence would write the whole L2 back)
+      __hip_atomic_store(part + ((k + 1) & 1) * kNBMax + o0 + kColQ * t, s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    }
+    column_barrier();
+    if (threadIdx.x == 0 &&
+        __hip_atomic_fetch_add(&st->arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == k * gridDim.x - 1)
+      __hip_atomic_store(&st->met, (unsigned)k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    load_next(k + 1);
+    if (threadIdx.x == 0) ok = grid_wait(st, (unsigned)k, spin);
+    column_barrier();
+    if (!ok) return;
+  }
+  const double sc = 1.0 / hn;
+#pragma unroll
+  for (int e = 0; e < E; ++e)
+    if (in[e]) vnext[index(e)] = sc * wr[e];
+  if (blockIdx.x == 0 && threadIdx.x == 0) gm_givens(st, G, m, j, itr, itrmax, rtol, hn, hist, hist_cap);
 }
 
 // y = H^-1 e on the leading mm x mm block (update_xVec, pcagmres.f90:1180-1192)
 __global__ void k_gm_backsub(GmState* st, GmArrays G, int m) {
-  if (st->done) return;
+  if (gm_halt(st)) return;
   if (threadIdx.x != 0 || blockIdx.x != 0) return;
   // the inner loop ran to completion: the reference's inner is m+1, mm = m
   if (!st->cycle_stop) st->inner = m + 1;
@@ -283,7 +449,7 @@ __global__ void k_gm_backsub(GmState* st, GmArrays G, int m) {
 // v0 = sum_{k=1..mm} y_k v_k  (sum_vec_FP64_CPU, pcagmres.f90:54-90)
 __global__ void __launch_bounds__(kNT) k_gm_sumvec(int n, const double* V, long ldv, double* __restrict__ v0,
                                                    const GmArrays G, int m, const GmState* st) {
-  if (st->done) return;
+  if (gm_halt(st)) return;
   const int mm = (int)G.y[m];
   for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
     double a = 0.0;
@@ -295,13 +461,13 @@ __global__ void __launch_bounds__(kNT) k_gm_sumvec(int n, const double* V, long 
 // x = x0 + x; end-of-cycle exit tests (pgmres.f90:455-475)
 __global__ void __launch_bounds__(kNT) k_gm_xadd(int n, double* __restrict__ x, const double* __restrict__ x0,
                                                  const GmState* st) {
-  if (st->done) return;
+  if (gm_halt(st)) return;
   for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x)
     x[i] = x0[i] + x[i];
 }
 
 __global__ void k_gm_endcycle(GmState* st, int itr, int itrmax) {
-  if (st->done || threadIdx.x != 0 || blockIdx.x != 0) return;
+  if (gm_halt(st) || threadIdx.x != 0 || blockIdx.x != 0) return;
   const int inner = st->inner;
   if (st->converged || itr + inner == itrmax) {
     st->done = 1;
@@ -309,6 +475,31 @@ __global__ void k_gm_endcycle(GmState* st, int itr, int itrmax) {
     st->niter = it < itrmax ? it : itrmax;
     st->iret = (itrmax <= itr) ? 1 : 0;
   }
+}
+
+// Launch of k_gm_column for vectors of n on this device: the kernel (null: not
+// used) and its workgroups.  It needs the whole column in registers: up to
+// eight elements a thread (n <= 2^21 on 256 CUs; more would spill at 1024
+// threads), and a device that launches cooperatively.
+struct ColumnLaunch {
+  const void* kern = nullptr;
+  int grid = 0;
+};
+ColumnLaunch column_launch(int n, int nb, int device) {
+  ColumnLaunch c;
+  int cu = 0, coop = 0;
+  if (hipDeviceGetAttribute(&cu, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess ||
+      hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, device) != hipSuccess || !coop || cu < 1)
+    return c;
+  const long ntiles = ((long)n + kNT - 1) / kNT;
+  const long rounds = (ntiles + nb - 1) / nb;
+  const int oq = nb <= kColQ * cu ? 1 : 2;
+  if (nb > 2 * kColQ * cu) return c;
+  c.grid = (nb + oq * kColQ - 1) / (oq * kColQ);
+  if (rounds <= 1) c.kern = oq == 1 ? (const void*)k_gm_column<1, 1> : (const void*)k_gm_column<2, 1>;
+  else if (rounds <= 2) c.kern = oq == 1 ? (const void*)k_gm_column<1, 2> : (const void*)k_gm_column<2, 2>;
+  else if (rounds <= 4) c.kern = oq == 1 ? (const void*)k_gm_column<1, 4> : (const void*)k_gm_column<2, 4>;
+  return c;
 }
 
 }  // namespace
@@ -366,6 +557,11 @@ int gmres_solve(Plan& P, double* x, const double* b, int itrmax, double rtol, do
   // cycle ends the solve) read as zero
   PARCEL_HIP_CHECK(hipMemsetAsync(P.hist.p, 0, sizeof(double) * (size_t)P.hist_cap, st));
   int launches = 0;
+  ColumnLaunch col = cgs ? ColumnLaunch() : column_launch(n, nb, P.device);
+  GmState before{};
+  // PARCEL_HIP_GM_SPIN: another bound on the wait (0: give up at once, to try the way back)
+  unsigned spin = kColSpin;
+  if (const char* e = std::getenv("PARCEL_HIP_GM_SPIN")) spin = (unsigned)std::strtoul(e, nullptr, 10);
   GmState* h = nullptr;
   PARCEL_HIP_CHECK(hipHostMalloc((void**)&h, sizeof(GmState), hipHostMallocDefault));
   const int* done = &S->done;
@@ -387,7 +583,20 @@ int gmres_solve(Plan& P, double* x, const double* b, int itrmax, double rtol, do
       precon_apply(P, vj, pv, nullptr, &S->cycle_stop);
       if (!cgs) {
         hipLaunchKernelGGL(k_gm_spmv, grid, block, 0, st, n, A, (const double*)pv, w, (const double*)V,
-                           gp, (const GmState*)S);
+                           gp, S);
+        if (col.kern) {
+          // partials of <w, v_1> in slot 0, the column's own in slots 1 and 2
+          const double *cw = w, *cV = V, *p0 = gp;
+          double *vnext = V + (long)j * ldv, *pp = gp + kNBMax, *hd = P.hist.p;
+          int cn = n, cnb = nb, cm = m, cj = j, citr = itr, cmax = itrmax, ccap = P.hist_cap;
+          long cld = ldv;
+          double ctol = rtol;
+          void* args[] = {&cn, &cw, &cV, &cld, &vnext, &p0,   &pp, &cnb, &S,
+                          &G,  &cm, &cj, &citr, &cmax, &ctol, &hd, &ccap, &spin};
+          PARCEL_HIP_CHECK(hipLaunchCooperativeKernel(col.kern, dim3(col.grid), dim3(kColT), args, 0, st));
+          launches += 3;
+          continue;
+        }
         for (int k = 1; k <= j; ++k) {
           const double* vk = V + (long)(k - 1) * ldv;
           const double* vnext = (k < j) ? V + (long)k * ldv : nullptr;
@@ -402,7 +611,7 @@ int gmres_solve(Plan& P, double* x, const double* b, int itrmax, double rtol, do
         launches += j + 3;
       } else {
         hipLaunchKernelGGL(k_gm_spmv, grid, block, 0, st, n, A, (const double*)pv, w, (const double*)nullptr,
-                           gp, (const GmState*)S);
+                           gp, S);
         for (int k0 = 1; k0 <= j; k0 += 8) {
           const int cnt = std::min(8, j - k0 + 1);
 #define PARCEL_CGS_DOTS(C)                                                                              \
@@ -437,6 +646,15 @@ int gmres_solve(Plan& P, double* x, const double* b, int itrmax, double rtol, do
     PARCEL_HIP_CHECK(hipGetLastError());
     PARCEL_HIP_CHECK(hipMemcpyAsync(h, S, sizeof(GmState), hipMemcpyDeviceToHost, st));
     PARCEL_HIP_CHECK(hipStreamSynchronize(st));
+    if (h->stuck) {
+      // the state as it was before this cycle (k_gm_init makes the first one's)
+      col.kern = nullptr;
+      if (itr > 1) PARCEL_HIP_CHECK(hipMemcpyAsync(S, &before, sizeof(GmState), hipMemcpyHostToDevice, st));
+      PARCEL_HIP_CHECK(hipStreamSynchronize(st));
+      itr -= m;
+      continue;
+    }
+    before = *h;
     if (h->done) break;
   }
   PARCEL_HIP_CHECK(hipEventRecord(ev1, st));
