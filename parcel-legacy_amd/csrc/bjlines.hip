@@ -37,8 +37,8 @@
 // 256 x 256 with the fused update 374 -> 366 us in the solve; 80 blocks of two
 // 160 x 160 planes D-ILU 813 -> 199 us; 256 blocks of 10 1/4 lines of 75 cells
 // D-ILU 136 -> 23 us.  Double-double, 32 blocks of three 96 x 96 planes ILU(0)
-// (level-scheduled before): 675 -> 350 us, bound by FP64 issue (six wavefronts
-// on four SIMDs).
+// (level-scheduled before): 675 -> 284 us (350 with Dekker's products), bound
+// by FP64 issue (six wavefronts on four SIMDs).
 #include <algorithm>
 #include <cstdlib>
 #include <type_traits>
@@ -166,6 +166,7 @@ struct LineArgs {
   const double* e[2][2];
   int nx;
   long nxy;
+  int wide;  // double-double: no fma products (a factor value is outside dd_fma_range)
 };
 
 // The couplings' stored order is fixed by the factor: the forward rows of
@@ -187,12 +188,67 @@ __host__ __device__ __forceinline__ dd dd_div_one(dd z) {
   return mkdd(h, l - (h - z.hi));
 }
 
+// dd_mul and dd_div with the error of the hi parts' product from one fma in
+// place of Dekker's split (2 operations for 17).  Both are that error exactly,
+// so the bits are the same, while the split does not overflow and no partial
+// product underflows: operands of [2^-480, 2^480] or 0 (a zero product gives
+// +0 both ways).  The host tests the factor against that range, the sweep
+// every value it produces (FmaRange), and a block with one outside is swept
+// again from its input with dd_mul and dd_div.
+__device__ __forceinline__ dd dd_mul_fma(dd a, dd b) {
+  const double t1h = a.hi * b.hi;
+  double t1l = fma(a.hi, b.hi, -t1h);
+  t1l = t1l + (a.hi * b.lo + a.lo * b.hi);
+  const double s1 = t1h + t1l;
+  t1l = t1l - (s1 - t1h);
+  return mkdd(s1, t1l);
+}
+__device__ __forceinline__ dd dd_div_fma(dd a, dd b) {
+  const double q1 = a.hi / b.hi;
+  double t1h = b.hi * q1;
+  double t1l = fma(b.hi, q1, -t1h);
+  t1l = t1l + (b.lo * q1);
+  double s1 = t1h + t1l;
+  t1l = t1l - (s1 - t1h);
+  t1h = s1;
+  s1 = a.hi - t1h;
+  const double r1 = s1 - a.hi;
+  double s2 = (a.hi - (s1 - r1)) - (t1h + r1);
+  s2 = s2 - t1l;
+  s2 = s2 + a.lo;
+  const double q2 = (s1 + s2) / b.hi;
+  const double h = q1 + q2;
+  return mkdd(h, q2 - (h - q1));
+}
+constexpr int kFmaLo = (1023 - 480) << 20, kFmaHi = (1023 + 480) << 20;  // high words of 2^-480 and 2^480
+inline bool dd_fma_range(double v) {
+  unsigned long long u;
+  __builtin_memcpy(&u, &v, 8);
+  const int t = (int)((u >> 32) & 0x7fffffff);
+  return (t >= kFmaLo && t < kFmaHi) || (u << 1) == 0;
+}
+// The smallest and largest magnitude seen, as high words less one: a zero
+// wraps to the largest unsigned and the smallest signed number, and a
+// subnormal whose high word is empty counts as 1.
+struct FmaRange {
+  unsigned lo = 0xffffffffu;
+  int hi = -1;
+  __device__ __forceinline__ void see(double v) {
+    const unsigned l = (unsigned)__double2loint(v);
+    const unsigned t = (((unsigned)__double2hiint(v) & 0x7fffffffu) | (l < 1u ? l : 1u)) - 1u;
+    lo = t < lo ? t : lo;
+    hi = (int)t > hi ? (int)t : hi;
+  }
+  __device__ __forceinline__ bool outside() const { return lo < (unsigned)(kFmaLo - 1) || hi >= kFmaHi - 1; }
+};
+
 // One sweep of a block.  NR: steps the factor operands are loaded ahead.
 // alphaf: the fused update's alpha, asked for once the first loads are out.
-template <bool FWD, int MODE, bool FUSED, bool PL, bool MULTI, int NV, int NR, class AF>
+template <bool FWD, int MODE, bool FUSED, bool PL, bool MULTI, int NV, int NR, bool FMA = false, class AF>
 __device__ __forceinline__ void line_sweep(const LineArgs& A, const LineBlock bk, const LineWave wv, int w, int W,
                                            const typename Num<NV>::Vec in, const typename Num<NV>::Vec out,
-                                           const typename Num<NV>::Vec q, AF alphaf, typename Num<NV>::L* lds) {
+                                           const typename Num<NV>::Vec q, AF alphaf, typename Num<NV>::L* lds,
+                                           FmaRange* rg = nullptr) {
   using N = Num<NV>;
   using V = typename N::V;
   constexpr bool kScale = !(FWD && MODE == BJ_ILU0);
@@ -343,7 +399,7 @@ __device__ __forceinline__ void line_sweep(const LineArgs& A, const LineBlock bk
       constexpr bool kAdd = !FWD && MODE == BJ_DILU;
       dd z = kAdd ? mkdd(0.0, 0.0) : a;
       auto term = [&](bool has, dd v, dd cf) {
-        const dd prod = dd_mul(v, cf);
+        const dd prod = FMA ? dd_mul_fma(v, cf) : dd_mul(v, cf);
         z = N::sel(has, kAdd ? dd_add(z, prod) : dd_sub(z, prod), z);
       };
       if constexpr (line_cell_first<FWD, MODE>()) {
@@ -355,10 +411,11 @@ __device__ __forceinline__ void line_sweep(const LineArgs& A, const LineBlock bk
         term(hl, yd, o.c.x);
         term(hc, yprev, o.c.y);
       }
-      if constexpr (MODE == BJ_ILU0) y = FWD ? dd_div_one(z) : dd_div(z, o.d);
+      if constexpr (MODE == BJ_ILU0) y = FWD ? dd_div_one(z) : FMA ? dd_div_fma(z, o.d) : dd_div(z, o.d);
       else y = FWD ? dd_mul(z, o.d) : dd_sub(a, dd_mul(o.d, z));
     }
     yprev = N::sel(on, y, N::num(kZero));
+    if constexpr (FMA) rg->see(yprev.hi);
     return yprev;
   };
   int ri = rin0 * 8 - sg * 64, ci = cin0 * 8 - 64;  // of in(-1)
@@ -451,7 +508,7 @@ __device__ __forceinline__ typename Num<NV>::Vec line_vec(const double* h, const
 template <int MODE, int NTH, bool PL, bool FUSED>
 __global__ void __launch_bounds__(NTH) k_bj_lines(LineArgs A, const double* rin, double* s, CGFuse fuse,
                                                   const int* skip) {
-  extern __shared__ double lds_lines[];
+  extern __shared__ __align__(16) double lds_lines[];
   __shared__ double sh[kWaves];
   constexpr bool MULTI = NTH > 64;
   constexpr int NR = NTH > 256 ? 8 : 16;
@@ -490,7 +547,7 @@ __global__ void __launch_bounds__(NTH) k_bj_lines(LineArgs A, const double* rin,
 template <int MODE, int NTH, bool PL>
 __global__ void __launch_bounds__(NTH) k_bj_lines_dd(LineArgs A, const double* rh, const double* rl, double* sh,
                                                      double* sl, const int* skip) {
-  extern __shared__ double lds_lines[];
+  extern __shared__ __align__(16) double lds_lines[];
   constexpr bool MULTI = NTH > 64;
   const int W = MULTI ? (int)(blockDim.x >> 6) : 1;
   const int w = MULTI ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
@@ -501,10 +558,24 @@ __global__ void __launch_bounds__(NTH) k_bj_lines_dd(LineArgs A, const double* r
   using Vec = Num<2>::Vec;
   const Vec vs = line_vec<2>(sh, sl, bk), vr = line_vec<2>(rh, rl, bk);
   dd16* lds = reinterpret_cast<dd16*>(lds_lines);
+  // lds_lines asks for 16-byte alignment because of this: 8 bytes off, the
+  // rings' 128-bit accesses took the apply from 284 to 502 us
+  __shared__ int outside;
+  if (threadIdx.x == 0) outside = 0;
   auto none = []() -> double { return 0.0; };
-  line_sweep<true, MODE, false, PL, MULTI, 2, 4>(A, bk, wf, w, W, vr, vs, vs, none, lds);
-  __syncthreads();  // forward values in memory before other threads' backward rows read them
-  line_sweep<false, MODE, false, PL, MULTI, 2, 4>(A, bk, wb, w, W, vs, vs, vs, none, lds);
+  auto sweeps = [&](auto fma, FmaRange* rg) {
+    line_sweep<true, MODE, false, PL, MULTI, 2, 4, decltype(fma)::value>(A, bk, wf, w, W, vr, vs, vs, none, lds, rg);
+    __syncthreads();  // forward values in memory before other threads' backward rows read them
+    line_sweep<false, MODE, false, PL, MULTI, 2, 4, decltype(fma)::value>(A, bk, wb, w, W, vs, vs, vs, none, lds, rg);
+  };
+  if (!A.wide) {
+    FmaRange rg;
+    sweeps(std::true_type(), &rg);
+    if (__any(rg.outside())) outside = 1;
+    __syncthreads();  // the flag, and the rings and stores before they are written again
+    if (!outside) return;
+  }
+  sweeps(std::false_type(), nullptr);
 }
 
 size_t line_lds_bytes(int W, int parts) { return sizeof(double) * (size_t)parts * (64 * (size_t)W + 1) * kLL; }
@@ -605,8 +676,8 @@ bool line_setup_at(Plan& P, const std::vector<BlockSweep>& F, const std::vector<
       ev[dir][q].assign((size_t)ne[dir] * (size_t)ents, 0.0);
     }
   const bool lo_on = P.M.dd_prec == 2;  // precision 1 applies the factors' hi parts only
-  int bad = 0;
-#pragma omp parallel for schedule(dynamic) reduction(| : bad)
+  int bad = 0, wide = 0;
+#pragma omp parallel for schedule(dynamic) reduction(| : bad, wide)
   for (int b = 0; b < nblk; ++b) {
     const Pieces& p = pc[b];
     const long z0 = (blo[b] / nx) / ny_plane;
@@ -651,6 +722,8 @@ bool line_setup_at(Plan& P, const std::vector<BlockSweep>& F, const std::vector<
           if (bad) break;
           c[dir][q][2 * e] = cell_first ? vc : vl;
           c[dir][q][2 * e + 1] = cell_first ? vl : vc;
+          if (pe == 2 && q == 0 && !(dd_fma_range(vc) && dd_fma_range(vl) && dd_fma_range(vp) && dd_fma_range(S.diag[i])))
+            wide = 1;
           const double dg = q ? (lo_on ? S.diag_lo[i] : 0.0) : S.diag[i];
           double* t = ev[dir][q].data() + (size_t)ne[dir] * e;
           if (pl) *t++ = vp;
@@ -674,6 +747,7 @@ bool line_setup_at(Plan& P, const std::vector<BlockSweep>& F, const std::vector<
   G.nxy = pl ? nxy : 0;
   G.waves = W;
   G.whole = whole && parts == 1;
+  G.wide = wide != 0;
   G.on = true;
   (void)n;
   return true;
@@ -691,6 +765,7 @@ LineArgs line_args(const LineBJ& G) {
     }
   A.nx = G.nx;
   A.nxy = G.nxy;
+  A.wide = G.wide ? 1 : 0;
   return A;
 }
 
@@ -775,7 +850,8 @@ void line_apply(Plan& P, const double* r, double* s, const CGFuse* fuse, const i
 void line_apply_dd(Plan& P, const double* rh, const double* rl, double* sh, double* sl, const int* skip) {
   const Precon& M = P.M;
   const LineBJ& G = M.line;
-  const LineArgs A = line_args(G);
+  LineArgs A = line_args(G);
+  if (rh == sh || rl == sl) A.wide = 1;  // no input to sweep again from
   const size_t shm = line_lds_bytes(G.waves, 2);
 #define PARCEL_LINE_K(MODE, NTH, PL) \
   launch_lines(k_bj_lines_dd<MODE, NTH, PL>, M.nblocks, G.waves, shm, P.stream, A, rh, rl, sh, sl, skip)

@@ -217,6 +217,7 @@ struct LineWave {
 struct LineBJ {
   bool on = false;
   bool whole = false;     // every block is whole grid lines (and whole planes when it couples planes)
+  bool wide = false;      // double-double: factor values beyond the range of the fma products
   int nx = 0;
   long nxy = 0;           // rows per plane (0: blocks do not couple planes)
   int waves = 1;          // wavefronts per workgroup

@@ -47,3 +47,33 @@ def test_ddcg_bit_exact(case, ilu, pp):
     assert np.array_equal(hist, ho)
     assert np.array_equal(xh.view(np.uint64), oh.view(np.uint64))
     assert np.array_equal(xl.view(np.uint64), ol.view(np.uint64))
+
+
+@pytest.mark.parametrize("ilu", [0, 1])
+@pytest.mark.parametrize("part", ["all", "one_row", "one_plane"])
+def test_values_beyond_the_fma_range(part, ilu):
+    # values below 2^-480 somewhere: the block is swept again with Dekker's
+    # products, whose partial products round where the fma's error would not
+    print("dd lines range", part, ilu, flush=True)
+    nx, ny, nz = 12, 96, 6
+    rp, col, val = ph.poisson3d_spd(nx, ny, nz)
+    n = rp.shape[0] - 1
+    b = ph.uniform(n, 92)
+    blo = b * 2.0 ** -56
+    sel = {"all": slice(None), "one_row": slice(700, 701), "one_plane": slice(nx * ny, 2 * nx * ny)}[part]
+    if part != "all":
+        b[: 2 * nx * ny] = 0.0
+        blo[: 2 * nx * ny] = 0.0
+        b[sel] = ph.uniform(n, 93)[sel]
+    down = 2.0 ** (-500 if part == "all" else -1000)  # "all": the norms stay above zero
+    b[sel] *= down
+    blo[sel] *= down
+    xh, xl = np.zeros(n), np.zeros(n)
+    hist, niter, iret = ph.ddcg(xh, xl, b, blo, rp, col, val, None, ipreflag=2, ILU_method=ilu, precon_thblock=3,
+                                itrmax=6, rtolmax=1e-30, PRECISION_A=1, PRECISION_b=2, PRECISION_x=2)
+    oh, ol, ho, no, io = orc.ddcg(rp, col, val, None, b, blo, ipreflag=2, ilu_method=ilu, nblocks=3, prec=2,
+                                  itrmax=6, rtol=1e-30)
+    assert (niter, iret) == (no, io)
+    assert np.array_equal(xh.view(np.uint64), oh.view(np.uint64))
+    assert np.array_equal(xl.view(np.uint64), ol.view(np.uint64))
+    assert np.array_equal(hist, ho)
