@@ -34,7 +34,7 @@
 // Measured, one apply, against the kernels before (a line form for whole lines
 // and planes with addresses selected per lane; level-scheduled sweeps for the
 // others): 64 blocks of two 128 x 128 planes ILU(0) 157 -> 92 us; 256 planes of
-// 256 x 256 with the fused update 374 -> 366 us in the solve; 80 blocks of two
+// 256 x 256 with the fused update 340 -> 313 us in the solve; 80 blocks of two
 // 160 x 160 planes D-ILU 813 -> 199 us; 256 blocks of 10 1/4 lines of 75 cells
 // D-ILU 136 -> 23 us.  Double-double, 32 blocks of three 96 x 96 planes ILU(0)
 // (level-scheduled before): 675 -> 284 us (350 with Dekker's products), bound
