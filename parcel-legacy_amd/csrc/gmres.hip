@@ -593,9 +593,14 @@ int gmres_solve(Plan& P, double* x, const double* b, int itrmax, double rtol, do
           double ctol = rtol;
           void* args[] = {&cn, &cw, &cV, &cld, &vnext, &p0,   &pp, &cnb, &S,
                           &G,  &cm, &cj, &citr, &cmax, &ctol, &hd, &ccap, &spin};
-          PARCEL_HIP_CHECK(hipLaunchCooperativeKernel(col.kern, dim3(col.grid), dim3(kColT), args, 0, st));
-          launches += 3;
-          continue;
+          if (hipLaunchCooperativeKernel(col.kern, dim3(col.grid), dim3(kColT), args, 0, st) == hipSuccess) {
+            launches += 3;
+            continue;
+          }
+          // refused (a GPU serves one process's cooperative launches at a time,
+          // and another one has it): this column and the rest step by step
+          (void)hipGetLastError();
+          col.kern = nullptr;
         }
         for (int k = 1; k <= j; ++k) {
           const double* vk = V + (long)(k - 1) * ldv;

@@ -4,6 +4,8 @@ owners per quarter workgroup, one, two and four tiles per owner, a last tile
 cut short, and a length whose column does not fit the registers), and the
 cycle run again with a kernel per step when the workgroups do not meet."""
 import os
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -48,3 +50,21 @@ def test_workgroups_that_do_not_meet(spin):
         _both(40, 40, 4, 400, 1e-9)
     finally:
         del os.environ["PARCEL_HIP_GM_SPIN"]
+
+
+def test_second_process():
+    # the first process's cooperative launches can keep a second one from its
+    # own: that one solves step by step, same bits
+    print("gmres column, second process", flush=True)
+    _both(40, 30, 5, 12)
+    code = ("import sys; sys.path.insert(0, %r); import numpy as np; import parcel_hip as ph; ph.init(0); "
+            "rp, c, v = ph.poisson2d(40, 30, -1.0); n = len(rp) - 1; x = np.zeros(n); "
+            "h, k, r = ph.dgmres(x, ph.uniform(n, 37), rp, c, v, GMRES_m=5, GMRES_GSflag=1, itrmax=12, "
+            "rtolmax=1e-12, ipreflag=1); print(x.tobytes().hex())" % os.path.dirname(os.path.abspath(ph.__file__)))
+    out = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=90)
+    assert out.returncode == 0, out.stdout + out.stderr
+    rp, col, val = ph.poisson2d(40, 30, -1.0)
+    n = rp.shape[0] - 1
+    x = np.zeros(n)
+    ph.dgmres(x, ph.uniform(n, 37), rp, col, val, GMRES_m=5, GMRES_GSflag=1, itrmax=12, rtolmax=1e-12, ipreflag=1)
+    assert out.stdout.split()[-1] == x.tobytes().hex()
