@@ -21,8 +21,10 @@ namespace parcel {
 namespace {
 
 struct BiState {
-  double bnorm, rnorm, c1, c2, c3, alpha, beta;
-  int itr, done, niter, iret;
+  double bnorm, rnorm, c1, c2, c3, alpha;
+  int itr;
+  int done;  // the iteration that ended the loop (0: none yet)
+  int niter, iret;
 };
 
 enum { BP_BB = 0, BP_RR0 = 1, BP_C2 = 2, BP_EV = 3, BP_VV = 4, BP_C1 = 5, BP_RR = 6 };
@@ -59,7 +61,7 @@ __global__ void __launch_bounds__(kNT) k_bi_init(const double* part, int nb, BiS
     st->bnorm = sqrt(bb);
     st->rnorm = sqrt(rr);
     st->c1 = rr;  // <r0,r0> with r0 = r: the same partials, the same order
-    st->c2 = st->c3 = st->alpha = st->beta = 0.0;
+    st->c2 = st->c3 = st->alpha = 0.0;
     st->itr = 0;
     st->done = 0;
     st->niter = 0;
@@ -119,13 +121,15 @@ __global__ void __launch_bounds__(kNT) k_bi_update(int n, double* __restrict__ x
   store_partials<2>(part, slots, acc, sh2);
 }
 
-// exit test and beta (pbicg.f90:590-625); p = r - beta c3 q + beta p.  (A
-// workgroup that starts after workgroup 0 has set `done` here returns at once,
-// as it would from its own exit test.)
+// exit test and beta (pbicg.f90:590-625) of iteration `it`; p = r - beta c3 q + beta p.
+// Workgroup 0 writes `done` = it while other wavefronts have yet to read it: they
+// test for an earlier iteration's exit only, so that all wavefronts of a workgroup
+// go through the reduction's barriers or none does, and leave by their own exit test.
 __global__ void __launch_bounds__(kNT) k_bi_p(int n, double* __restrict__ p, const double* __restrict__ r,
                                               const double* __restrict__ q, const double* part, int nb, BiState* st,
-                                              int itrmax, double rtol) {
-  if (st->done) return;
+                                              int it, int itrmax, double rtol) {
+  const int done = st->done;
+  if (done != 0 && done < it) return;
   __shared__ double sh2[kWaves * 2];
   double c1, rr;
   reduce_part2(part + BP_C1 * kNBMax, part + BP_RR * kNBMax, nb, sh2, c1, rr);
@@ -137,11 +141,9 @@ __global__ void __launch_bounds__(kNT) k_bi_p(int n, double* __restrict__ p, con
     st->rnorm = rnorm;
     st->c1 = c1;
     if (last) {
-      st->done = 1;
+      st->done = it;
       st->niter = itr;                     // min(itrmax, itr)
       st->iret = (itrmax <= itr) ? 1 : 0;  // pbicg.f90:672-676
-    } else {
-      st->beta = beta;
     }
   }
   if (last) return;
@@ -210,7 +212,7 @@ int bicg_solve(Plan& P, double* x, const double* b, int itrmax, double rtol, dou
       hipLaunchKernelGGL(k_bi_update, grid, block, 0, st, n, x, (const double*)pp, (const double*)pe, r,
                          (const double*)e, (const double*)v, (const double*)r0, part, S);
       hipLaunchKernelGGL(k_bi_p, grid, block, 0, st, n, p, (const double*)r, (const double*)q, (const double*)part, nb,
-                         S, itrmax, rtol);
+                         S, enq + j + 1, itrmax, rtol);
       launches += 7;
     }
     PARCEL_HIP_CHECK(hipGetLastError());
