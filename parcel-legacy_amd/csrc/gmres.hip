@@ -270,7 +270,11 @@ __device__ void gm_givens(GmState* st, const GmArrays& G, int m, int j, int itr,
 __global__ void __launch_bounds__(kNT) k_gm_norm(int n, const double* __restrict__ w, double* __restrict__ vnext,
                                                  const double* part, int nb_prod, GmState* st, GmArrays G, int m,
                                                  int j, int itr, int itrmax, double rtol, double* hist, int hist_cap) {
-  if (gm_skip(st)) return;
+  // once per workgroup: workgroup 0 may set cycle_stop (gm_givens) while others start
+  __shared__ int skip;
+  if (threadIdx.x == 0) skip = gm_skip(st);
+  __syncthreads();
+  if (skip) return;
   __shared__ double sh[kWaves];
   const double hn = sqrt(reduce_part(part, nb_prod, sh));
   const double sc = 1.0 / hn;
@@ -329,10 +333,15 @@ __global__ void __launch_bounds__(kColT) k_gm_column(int n, const double* __rest
                                                      double* vnext, const double* part0, double* part, int nb,
                                                      GmState* st, GmArrays G, int m, int j, int itr, int itrmax,
                                                      double rtol, double* hist, int hist_cap, unsigned spin) {
-  if (gm_skip(st)) return;  // the state of earlier launches: the same in every workgroup
   constexpr int E = OQ * RD;
   __shared__ double sh[OQ][kColT / 64], shr[kWaves];
+  // Once per workgroup, so that its wavefronts keep together at the barriers:
+  // another one may set `stuck` meanwhile (this workgroup then leaves here or
+  // from its wait).
   __shared__ int ok;
+  if (threadIdx.x == 0) ok = !gm_skip(st);
+  column_barrier();
+  if (!ok) return;
   const int q = threadIdx.x / kNT, t = threadIdx.x % kNT, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   // element e = (mo, r): owner o0 + kColQ mo, its tile r
   const int o0 = blockIdx.x * (OQ * kColQ) + q;

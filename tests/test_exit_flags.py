@@ -32,7 +32,7 @@ def closure(body, helpers):
     return text
 
 
-@pytest.mark.parametrize("name", ["bicg.hip", "ddcg.hip", "cg_kernels.hpp"])
+@pytest.mark.parametrize("name", ["bicg.hip", "gmres.hip", "ddcg.hip", "cg_kernels.hpp"])
 def test_no_wavefront_tests_a_field_its_own_launch_writes(name):
     src = re.sub(r"//[^\n]*|__launch_bounds__\(\w+\)", "", open(os.path.join(CSRC, name)).read())
     helpers = dict(functions(src, r"__device__"))
