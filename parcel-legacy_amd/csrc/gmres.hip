@@ -511,6 +511,13 @@ ColumnLaunch column_launch(int n, int nb, int device) {
   return c;
 }
 
+// Whether a cooperative launch was refused rather than failed: another process
+// has the GPU's cooperative launches (one process's are served at a time), or
+// the grid does not fit the compute units that this process may use.
+bool coop_refused(hipError_t rc) {
+  return rc == hipErrorIllegalState || rc == hipErrorCooperativeLaunchTooLarge || rc == hipErrorNotSupported;
+}
+
 }  // namespace
 
 int gmres_solve(Plan& P, double* x, const double* b, int itrmax, double rtol, double* hist_host, int* niter,
@@ -602,12 +609,14 @@ int gmres_solve(Plan& P, double* x, const double* b, int itrmax, double rtol, do
           double ctol = rtol;
           void* args[] = {&cn, &cw, &cV, &cld, &vnext, &p0,   &pp, &cnb, &S,
                           &G,  &cm, &cj, &citr, &cmax, &ctol, &hd, &ccap, &spin};
-          if (hipLaunchCooperativeKernel(col.kern, dim3(col.grid), dim3(kColT), args, 0, st) == hipSuccess) {
+          PARCEL_HIP_CHECK(hipGetLastError());  // of the launches so far: a refusal is cleared below
+          const hipError_t rc = hipLaunchCooperativeKernel(col.kern, dim3(col.grid), dim3(kColT), args, 0, st);
+          if (rc == hipSuccess) {
             launches += 3;
             continue;
           }
-          // refused (a GPU serves one process's cooperative launches at a time,
-          // and another one has it): this column and the rest step by step
+          if (!coop_refused(rc)) PARCEL_HIP_CHECK(rc);
+          // this column and the rest step by step
           (void)hipGetLastError();
           col.kern = nullptr;
         }

@@ -1,8 +1,11 @@
 """GMRES(m) with MGS, a whole column per launch (k_gm_column): bit for bit
 against the oracle at the sizes where its launch changes shape (one and two
 owners per quarter workgroup, one, two and four tiles per owner, a last tile
-cut short, and a length whose column does not fit the registers), and the
-cycle run again with a kernel per step when the workgroups do not meet."""
+cut short, and a length whose column does not fit the registers), the cycle
+run again with a kernel per step when the workgroups do not meet, and the
+steps taken when the launch is refused.  The launches that a solve counts say
+which way its columns went: a restart cycle of m columns takes 8 and three a
+column resident, 8 and j + 3 for column j step by step."""
 import os
 import subprocess
 import sys
@@ -21,13 +24,24 @@ def _init():
     ph.init(0)
 
 
-def _both(nx, ny, m, itrmax, rtol=1e-12):
+def _cycles(launches, m, way):
+    """Restart cycles that `launches` make (0: not a whole number) when all
+    columns run `way`; "again": the first cycle resident, then all step by step."""
+    resident, steps = 8 + 3 * m, 8 + 3 * m + m * (m + 1) // 2
+    rest = launches - 1 - (resident + 1 if way == "again" else 0)
+    per = resident if way == "resident" else steps
+    return rest // per if rest > 0 and rest % per == 0 else 0
+
+
+def _both(nx, ny, m, itrmax, rtol=1e-12, way="resident"):
     rp, col, val = ph.poisson2d(nx, ny, -1.0)
     n = rp.shape[0] - 1
     b = ph.uniform(n, 37)
     x = np.zeros(n)
-    hist, niter, iret = ph.dgmres(x, b, rp, col, val, GMRES_m=m, GMRES_GSflag=1, itrmax=itrmax, rtolmax=rtol,
-                                  ipreflag=1)
+    with ph.Plan(rp, col, val, solver=ph.SOLVER_GMRES, GMRES_m=m, GMRES_GSflag=1, ipreflag=1) as P:
+        hist, niter, iret = P.solve(x, b, itrmax, rtol)
+        launches = P.stats()["launches"]
+    assert 1 <= _cycles(launches, m, way) <= niter // m + 1, (launches, niter)
     xo, ho, no, io = orc.gmres(rp, col, val, b, ipreflag=1, ilu_method=1, nblocks=1, itrmax=itrmax, rtol=rtol, m=m,
                                gsflag=1)
     assert (niter, iret) == (no, io)
@@ -38,7 +52,7 @@ def _both(nx, ny, m, itrmax, rtol=1e-12):
                                    (1449, 1449)])
 def test_column_bit_exact(nx, ny):
     print("gmres column", nx, ny, flush=True)
-    _both(nx, ny, 5, 12)
+    _both(nx, ny, 5, 12, way="resident" if nx * ny <= 2 ** 21 else "steps")
 
 
 @pytest.mark.parametrize("spin", ["0", "3"])
@@ -46,25 +60,28 @@ def test_workgroups_that_do_not_meet(spin):
     print("gmres column spin", spin, flush=True)
     os.environ["PARCEL_HIP_GM_SPIN"] = spin
     try:
-        _both(300, 301, 6, 20)
-        _both(40, 40, 4, 400, 1e-9)
+        _both(300, 301, 6, 20, way="again")
+        _both(40, 40, 4, 400, 1e-9, way="again")
     finally:
         del os.environ["PARCEL_HIP_GM_SPIN"]
 
 
 def test_second_process():
-    # the first process's cooperative launches can keep a second one from its
-    # own: that one solves step by step, same bits
+    # the first process's cooperative launches keep a second one from its own:
+    # that one solves step by step, same bits
     print("gmres column, second process", flush=True)
     _both(40, 30, 5, 12)
     code = ("import sys; sys.path.insert(0, %r); import numpy as np; import parcel_hip as ph; ph.init(0); "
             "rp, c, v = ph.poisson2d(40, 30, -1.0); n = len(rp) - 1; x = np.zeros(n); "
-            "h, k, r = ph.dgmres(x, ph.uniform(n, 37), rp, c, v, GMRES_m=5, GMRES_GSflag=1, itrmax=12, "
-            "rtolmax=1e-12, ipreflag=1); print(x.tobytes().hex())" % os.path.dirname(os.path.abspath(ph.__file__)))
+            "P = ph.Plan(rp, c, v, solver=ph.SOLVER_GMRES, GMRES_m=5, GMRES_GSflag=1, ipreflag=1); "
+            "P.solve(x, ph.uniform(n, 37), 12, 1e-12); print(P.stats()['launches'], x.tobytes().hex())"
+            % os.path.dirname(os.path.abspath(ph.__file__)))
     out = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=90)
     assert out.returncode == 0, out.stdout + out.stderr
+    launches, xhex = out.stdout.split()[-2:]
+    assert _cycles(int(launches), 5, "steps") == 2
     rp, col, val = ph.poisson2d(40, 30, -1.0)
     n = rp.shape[0] - 1
     x = np.zeros(n)
     ph.dgmres(x, ph.uniform(n, 37), rp, col, val, GMRES_m=5, GMRES_GSflag=1, itrmax=12, rtolmax=1e-12, ipreflag=1)
-    assert out.stdout.split()[-1] == x.tobytes().hex()
+    assert xhex == x.tobytes().hex()
