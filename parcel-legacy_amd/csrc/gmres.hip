@@ -19,6 +19,7 @@
 //             x0 = M^-1 v0 ; x = x0 + x
 // The small dense operations (Givens, back substitution) use plain
 // multiply/add as written in the reference, with no contraction.
+#include <atomic>
 #include <chrono>
 #include <cmath>
 #include <cstdlib>
@@ -511,6 +512,25 @@ ColumnLaunch column_launch(int n, int nb, int device) {
   return c;
 }
 
+// A refused attempt costs 37 ms (the runtime asks for the GPU's cooperative
+// queue and gives up), a small solve 2 to 5: for two seconds after a refusal
+// the device is not asked again by this process.  Nanoseconds of the steady
+// clock per device; any thread may read or write them.
+constexpr int kCoopDevices = 64;
+constexpr long long kCoopPause = 2000000000;
+std::atomic<long long> coop_after[kCoopDevices];
+long long steady_ns() {
+  return std::chrono::duration_cast<std::chrono::nanoseconds>(std::chrono::steady_clock::now().time_since_epoch())
+      .count();
+}
+bool coop_paused(int device) {
+  return device >= 0 && device < kCoopDevices && steady_ns() < coop_after[device].load(std::memory_order_relaxed);
+}
+void coop_pause(int device) {
+  if (device >= 0 && device < kCoopDevices)
+    coop_after[device].store(steady_ns() + kCoopPause, std::memory_order_relaxed);
+}
+
 // Whether a cooperative launch was refused rather than failed: another process
 // has the GPU's cooperative launches (one process's are served at a time), or
 // the grid does not fit the compute units that this process may use.
@@ -573,7 +593,7 @@ int gmres_solve(Plan& P, double* x, const double* b, int itrmax, double rtol, do
   // cycle ends the solve) read as zero
   PARCEL_HIP_CHECK(hipMemsetAsync(P.hist.p, 0, sizeof(double) * (size_t)P.hist_cap, st));
   int launches = 0;
-  ColumnLaunch col = cgs ? ColumnLaunch() : column_launch(n, nb, P.device);
+  ColumnLaunch col = cgs || coop_paused(P.device) ? ColumnLaunch() : column_launch(n, nb, P.device);
   GmState before{};
   // PARCEL_HIP_GM_SPIN: another bound on the wait (0: give up at once, to try the way back)
   unsigned spin = kColSpin;
@@ -618,6 +638,7 @@ int gmres_solve(Plan& P, double* x, const double* b, int itrmax, double rtol, do
           if (!coop_refused(rc)) PARCEL_HIP_CHECK(rc);
           // this column and the rest step by step
           (void)hipGetLastError();
+          coop_pause(P.device);
           col.kern = nullptr;
         }
         for (int k = 1; k <= j; ++k) {

@@ -24,16 +24,20 @@ def _init():
     ph.init(0)
 
 
-def _cycles(launches, m, way):
-    """Restart cycles that `launches` make (0: not a whole number) when all
-    columns run `way`; "again": the first cycle resident, then all step by step."""
+def _cycles(launches, m):
+    """(resident, step by step) restart cycles that a solve's launches make: all
+    of one kind, or resident ones up to a cycle that ran again by steps (the
+    first one's restart makes the state again: one launch more)."""
     resident, steps = 8 + 3 * m, 8 + 3 * m + m * (m + 1) // 2
-    rest = launches - 1 - (resident + 1 if way == "again" else 0)
-    per = resident if way == "resident" else steps
-    return rest // per if rest > 0 and rest % per == 0 else 0
+    for a in range(launches // resident + 1):
+        for again in ((0, 1) if a == 1 else (0,)):
+            rest = launches - 1 - again - a * resident
+            if rest >= 0 and rest % steps == 0 and (a == 0 or rest == 0 or a > 1 or again):
+                return a, rest // steps
+    return None
 
 
-def _both(nx, ny, m, itrmax, rtol=1e-12, way="resident"):
+def _both(nx, ny, m, itrmax, rtol=1e-12, way=None):
     rp, col, val = ph.poisson2d(nx, ny, -1.0)
     n = rp.shape[0] - 1
     b = ph.uniform(n, 37)
@@ -41,7 +45,8 @@ def _both(nx, ny, m, itrmax, rtol=1e-12, way="resident"):
     with ph.Plan(rp, col, val, solver=ph.SOLVER_GMRES, GMRES_m=m, GMRES_GSflag=1, ipreflag=1) as P:
         hist, niter, iret = P.solve(x, b, itrmax, rtol)
         launches = P.stats()["launches"]
-    assert 1 <= _cycles(launches, m, way) <= niter // m + 1, (launches, niter)
+    a, b_ = _cycles(launches, m)
+    assert way is None or {"resident": a > 0 and b_ == 0, "steps": a == 0, "again": a > 0 and b_ > 0}[way], (a, b_)
     xo, ho, no, io = orc.gmres(rp, col, val, b, ipreflag=1, ilu_method=1, nblocks=1, itrmax=itrmax, rtol=rtol, m=m,
                                gsflag=1)
     assert (niter, iret) == (no, io)
@@ -60,26 +65,31 @@ def test_workgroups_that_do_not_meet(spin):
     print("gmres column spin", spin, flush=True)
     os.environ["PARCEL_HIP_GM_SPIN"] = spin
     try:
-        _both(300, 301, 6, 20, way="again")
-        _both(40, 40, 4, 400, 1e-9, way="again")
+        # (with 89 workgroups one always polls too early; two may be in time)
+        _both(300, 301, 6, 20, way="again" if spin == "0" else None)
+        _both(40, 40, 4, 400, 1e-9)
     finally:
         del os.environ["PARCEL_HIP_GM_SPIN"]
 
 
 def test_second_process():
     # the first process's cooperative launches keep a second one from its own:
-    # that one solves step by step, same bits
+    # that one solves step by step, same bits, and does not ask again in every
+    # solve (an attempt that is refused takes some 37 ms, a solve a few)
     print("gmres column, second process", flush=True)
-    _both(40, 30, 5, 12)
-    code = ("import sys; sys.path.insert(0, %r); import numpy as np; import parcel_hip as ph; ph.init(0); "
+    _both(40, 30, 5, 12, way="resident")
+    code = ("import sys, time; sys.path.insert(0, %r); import numpy as np; import parcel_hip as ph; ph.init(0); "
             "rp, c, v = ph.poisson2d(40, 30, -1.0); n = len(rp) - 1; x = np.zeros(n); "
             "P = ph.Plan(rp, c, v, solver=ph.SOLVER_GMRES, GMRES_m=5, GMRES_GSflag=1, ipreflag=1); "
-            "P.solve(x, ph.uniform(n, 37), 12, 1e-12); print(P.stats()['launches'], x.tobytes().hex())"
+            "b = ph.uniform(n, 37); tm = [time.perf_counter()]\n"
+            "for k in range(6): x[:] = 0; P.solve(x, b, 12, 1e-12); tm.append(time.perf_counter())\n"
+            "print(tm[1] - tm[0], min(np.diff(tm[1:])), P.stats()['launches'], x.tobytes().hex())"
             % os.path.dirname(os.path.abspath(ph.__file__)))
     out = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=90)
     assert out.returncode == 0, out.stdout + out.stderr
-    launches, xhex = out.stdout.split()[-2:]
-    assert _cycles(int(launches), 5, "steps") == 2
+    first, later, launches, xhex = out.stdout.split()[-4:]
+    assert float(later) < 0.5 * float(first)
+    assert _cycles(int(launches), 5) == (0, 2)
     rp, col, val = ph.poisson2d(40, 30, -1.0)
     n = rp.shape[0] - 1
     x = np.zeros(n)
