@@ -512,6 +512,17 @@ ColumnLaunch column_launch(int n, int nb, int device) {
   return c;
 }
 
+// Whether column j of n rows goes to k_gm_column.  A step there saves most of
+// k_gm_mgs's passes over w and v_k but has a meeting to pay for, and a
+// cooperative launch some 25 us more than a plain one.  Microseconds a step,
+// k_gm_mgs / k_gm_column: 3.0 / 2.2 at 8^3 rows, 3.9 / 3.5 at 48^3, 5.1 / 5.0 at
+// 64^3, 6.5 / 5.9 at 80^3, 8.2 / 6.3 at 96^3, 11.4 / 6.8 at 112^3, 14.1 / 6.4 at
+// 128^3: from 450,000 rows on a step gains about 4.7 us per million rows more,
+// and j of them have to outweigh the launch.  The column kernel in every column
+// took 1.2 to 1.6 times the step kernels' time on all sizes up to 64^3.
+// PARCEL_HIP_GM_COLUMN=1 takes it for every column that fits, =0 for none.
+bool column_pays(int n, int j) { return (long)j * (n - 450000L) >= 8000000L; }
+
 // A refused attempt costs 37 ms (the runtime asks for the GPU's cooperative
 // queue and gives up), a small solve 2 to 5: for two seconds after a refusal
 // the device is not asked again by this process.  Nanoseconds of the steady
@@ -594,6 +605,8 @@ int gmres_solve(Plan& P, double* x, const double* b, int itrmax, double rtol, do
   PARCEL_HIP_CHECK(hipMemsetAsync(P.hist.p, 0, sizeof(double) * (size_t)P.hist_cap, st));
   int launches = 0;
   ColumnLaunch col = cgs || coop_paused(P.device) ? ColumnLaunch() : column_launch(n, nb, P.device);
+  int forced = -1;
+  if (const char* e = std::getenv("PARCEL_HIP_GM_COLUMN")) forced = e[0] == '1' ? 1 : e[0] == '0' ? 0 : -1;
   GmState before{};
   // PARCEL_HIP_GM_SPIN: another bound on the wait (0: give up at once, to try the way back)
   unsigned spin = kColSpin;
@@ -620,7 +633,7 @@ int gmres_solve(Plan& P, double* x, const double* b, int itrmax, double rtol, do
       if (!cgs) {
         hipLaunchKernelGGL(k_gm_spmv, grid, block, 0, st, n, A, (const double*)pv, w, (const double*)V,
                            gp, S);
-        if (col.kern) {
+        if (col.kern && (forced < 0 ? column_pays(n, j) : forced == 1)) {
           // partials of <w, v_1> in slot 0, the column's own in slots 1 and 2
           const double *cw = w, *cV = V, *p0 = gp;
           double *vnext = V + (long)j * ldv, *pp = gp + kNBMax, *hd = P.hist.p;

@@ -3,7 +3,9 @@ against the oracle at the sizes where its launch changes shape (one and two
 owners per quarter workgroup, one, two and four tiles per owner, a last tile
 cut short, and a length whose column does not fit the registers), the cycle
 run again with a kernel per step when the workgroups do not meet, and the
-steps taken when the launch is refused.  The launches that a solve counts say
+steps taken when the launch is refused.  PARCEL_HIP_GM_COLUMN=1 sends every
+column that fits there, as the rule on sizes sends the late columns of long
+vectors; one case runs by the rule.  The launches that a solve counts say
 which way its columns went: a restart cycle of m columns takes 8 and three a
 column resident, 8 and j + 3 for column j step by step."""
 import os
@@ -22,6 +24,9 @@ pytestmark = pytest.mark.gpu
 @pytest.fixture(scope="module", autouse=True)
 def _init():
     ph.init(0)
+    os.environ["PARCEL_HIP_GM_COLUMN"] = "1"
+    yield
+    del os.environ["PARCEL_HIP_GM_COLUMN"]
 
 
 def _cycles(launches, m):
@@ -45,12 +50,14 @@ def _both(nx, ny, m, itrmax, rtol=1e-12, way=None):
     with ph.Plan(rp, col, val, solver=ph.SOLVER_GMRES, GMRES_m=m, GMRES_GSflag=1, ipreflag=1) as P:
         hist, niter, iret = P.solve(x, b, itrmax, rtol)
         launches = P.stats()["launches"]
-    a, b_ = _cycles(launches, m)
-    assert way is None or {"resident": a > 0 and b_ == 0, "steps": a == 0, "again": a > 0 and b_ > 0}[way], (a, b_)
+    if way:
+        a, c = _cycles(launches, m)
+        assert {"resident": a > 0 and c == 0, "steps": a == 0, "again": a > 0 and c > 0}[way], (a, c)
     xo, ho, no, io = orc.gmres(rp, col, val, b, ipreflag=1, ilu_method=1, nblocks=1, itrmax=itrmax, rtol=rtol, m=m,
                                gsflag=1)
     assert (niter, iret) == (no, io)
     assert np.array_equal(hist, ho) and np.array_equal(x, xo)
+    return launches
 
 
 @pytest.mark.parametrize("nx,ny", [(7, 5), (16, 16), (511, 511), (513, 513), (724, 725), (1023, 1024), (1201, 1201),
@@ -70,6 +77,21 @@ def test_workgroups_that_do_not_meet(spin):
         _both(40, 40, 4, 400, 1e-9)
     finally:
         del os.environ["PARCEL_HIP_GM_SPIN"]
+
+
+@pytest.mark.parametrize("nx,ny,m", [(40, 50, 8), (750, 700, 8), (1023, 1024, 16), (1448, 1448, 6)])
+def test_columns_by_the_rule(nx, ny, m):
+    # short vectors by steps alone, longer ones by steps up to the column from
+    # which the resident kernel pays, inside one restart cycle
+    print("gmres columns by the rule", nx, ny, m, flush=True)
+    first = next((j for j in range(1, m + 1) if j * (nx * ny - 450000) >= 8000000), m + 1)
+    os.environ["PARCEL_HIP_GM_COLUMN"] = "rule"
+    try:
+        launches = _both(nx, ny, m, m)
+    finally:
+        os.environ["PARCEL_HIP_GM_COLUMN"] = "1"
+    assert launches == 1 + 8 + sum(3 + (j if j < first else 0) for j in range(1, m + 1))
+    assert nx * ny < 10 ** 6 or 1 < first <= m
 
 
 def test_second_process():
