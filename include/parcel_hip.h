@@ -109,9 +109,9 @@ typedef struct parcel_hip_stats {
   int vec_calls;
   /* preconditioner structure */
   int bj_blocks;
-  int bj_levels_fwd;
-  int bj_levels_bwd;
-  long bj_entries;         /* stored factor entries (both sweeps, with padding) */
+  int bj_levels_fwd;       /* dependency levels of the blocks' sweeps, summed over the blocks */
+  int bj_levels_bwd;       /* (of the factor: also where the apply does not go level by level) */
+  long bj_entries;         /* stored off-diagonal factor entries (both sweeps, with padding) */
   long bj_nnz_l;           /* off-diagonal entries read by the forward sweep */
   long bj_nnz_u;           /* off-diagonal entries read by the backward sweep */
   /* mixed-precision refinement (PARCEL_SOLVER_CG_MIXED) */
@@ -121,9 +121,8 @@ typedef struct parcel_hip_stats {
   int spmv_stencil;        /* 1: the CG kernel reads the matrix as a symmetric 5/7-point stencil (4 arrays) */
   long sell_entries;       /* stored SELL-64 entries (padding and the long rows' overflow included) */
   long sell_overflow;      /* entries of long rows kept after the slices (0: none) */
-  int bj_lines;            /* 1: the FP64 block-Jacobi apply runs as line wavefronts over blocks of whole
-                              grid lines or planes (blocks that cut a line or a plane run the same kernel
-                              where at most eight wavefronts hold their lines, and report 0) */
+  int bj_lines;            /* 1: the FP64 or double-double block-Jacobi apply runs as line wavefronts
+                              (0: level by level) */
 } parcel_hip_stats;
 
 /* --- library life cycle: PARCEL_Init / PARCEL_Free (src/c_krylov_wrapper.f90:6-22) */

@@ -623,7 +623,7 @@ bool line_setup_at(Plan& P, const std::vector<BlockSweep>& F, const std::vector<
   const bool ilu0 = P.M.mode == BJ_ILU0;
   std::vector<Pieces> pc(nblk);
   int W = 1;
-  bool pl = false, whole = true;
+  bool pl = false;
   for (int b = 0; b < nblk; ++b) {
     if (bhi[b] <= blo[b] || (long)(bhi[b] - blo[b]) * 8 >= (1L << 31)) return false;
     pc[b] = pieces_of(blo[b], bhi[b], nx, ny_plane, nxy);
@@ -631,8 +631,6 @@ bool line_setup_at(Plan& P, const std::vector<BlockSweep>& F, const std::vector<
     if (waves > 8) return false;
     W = std::max(W, (int)waves);
     pl = pl || pc[b].coupled;
-    const long unit = pc[b].coupled ? nxy : nx;
-    if (blo[b] % unit || bhi[b] % unit) whole = false;
   }
   if (line_lds_bytes(W, parts) > kLdsMax) return false;
   std::vector<LineBlock> blk(nblk);
@@ -746,7 +744,7 @@ bool line_setup_at(Plan& P, const std::vector<BlockSweep>& F, const std::vector<
   G.nx = X;
   G.nxy = pl ? nxy : 0;
   G.waves = W;
-  G.whole = whole && parts == 1;
+  G.entries = (pl ? 3 : 2) * ents;
   G.wide = wide != 0;
   G.on = true;
   (void)n;

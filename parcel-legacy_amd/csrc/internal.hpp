@@ -216,11 +216,11 @@ struct LineWave {
 };
 struct LineBJ {
   bool on = false;
-  bool whole = false;     // every block is whole grid lines (and whole planes when it couples planes)
   bool wide = false;      // double-double: factor values beyond the range of the fma products
   int nx = 0;
   long nxy = 0;           // rows per plane (0: blocks do not couple planes)
   int waves = 1;          // wavefronts per workgroup
+  long entries = 0;       // coupling slots a sweep stores
   DevBuf<LineBlock> blk;
   DevBuf<LineWave> fw, bw;         // waves per block each
   DevBuf<double> c[2][2];          // [forward, backward][hi, lo]: line and cell couplings per entry

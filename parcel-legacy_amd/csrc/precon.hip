@@ -436,8 +436,9 @@ void pack_sweep(const std::vector<BlockSweep>& blocks, const std::vector<int>& b
   PARCEL_HIP_CHECK(hipStreamSynchronize(st));
 }
 
-// The counts pack_sweep reports, for sweeps whose level form is not built.
-void count_sweep(const std::vector<BlockSweep>& blocks, int padk, Sweep& S) {
+// The counts pack_sweep reports, for sweeps that run as line wavefronts with
+// `entries` coupling slots and whose level form is not built.
+void count_sweep(const std::vector<BlockSweep>& blocks, int padk, long entries, Sweep& S) {
   long rows = 0, real = 0;
   int nlev = 0;
   for (const BlockSweep& B : blocks) {
@@ -448,7 +449,7 @@ void count_sweep(const std::vector<BlockSweep>& blocks, int padk, Sweep& S) {
   if (rows * padk > 0x7fffffffL)
     throw hip_error("block-Jacobi factor too large for int32 offsets", PARCEL_HIP_ERR_UNSUPPORTED);
   S.nlev = nlev;
-  S.entries = rows * padk;
+  S.entries = entries;
   S.real_entries = real;
 }
 
@@ -914,8 +915,8 @@ void precon_setup(Plan& P) {
           maxw = std::max(maxw, S->lev_start[l + 1] - S->lev_start[l]);
     M.nth = maxw <= 256 ? 256 : maxw <= 512 ? 512 : 1024;
     if (P.prm.solver != PARCEL_SOLVER_CG_MIXED && line_setup(P, F, B, blo, bhi, 1)) {
-      count_sweep(F, apply_k(kmax), M.fwd);
-      count_sweep(B, apply_k(kmax), M.bwd);
+      count_sweep(F, apply_k(kmax), M.line.entries, M.fwd);
+      count_sweep(B, apply_k(kmax), M.line.entries, M.bwd);
     } else {
       pack_sweep(F, blo, M.fwd, kRingBudget, apply_k(kmax), M.nth, P.stream);
       pack_sweep(B, blo, M.bwd, kRingBudget, apply_k(kmax), M.nth, P.stream);
@@ -1342,8 +1343,8 @@ void precon_setup_dd(Plan& P, int prec) {
     M.nth = maxw <= 256 ? 256 : 512;
     bool fast = maxw <= 512 && kk <= kKR;
     if (line_setup(P, F, B, blo, bhi, 2)) {
-      count_sweep(F, fast ? kk : kmax, M.fwd);
-      count_sweep(B, fast ? kk : kmax, M.bwd);
+      count_sweep(F, fast ? kk : kmax, M.line.entries, M.fwd);
+      count_sweep(B, fast ? kk : kmax, M.line.entries, M.bwd);
     } else {
       if (fast) {
         pack_sweep(F, blo, M.fwd, kRingBudget, kk, M.nth, P.stream);

@@ -1,5 +1,5 @@
 """GPU parity of the line-wavefront form of the FP64 block-Jacobi apply
-(precon.hip: line_setup, k_bj_lines) through the C ABI.
+(bjlines.hip: line_setup, k_bj_lines) through the C ABI.
 
 When every block is whole grid lines (strips of one plane, or whole planes)
 and its ILU(0) / D-ILU factor rows couple only to the neighbouring cell of
@@ -130,9 +130,16 @@ def test_nonsymmetric_solvers_bit_exact(case):
     (lambda: ph.poisson3d_spd(16, 16, 16), 3),    # blocks that cut a plane
     (lambda: ph.poisson2d(64, 64, -1.0), 7),      # blocks that cut a line
 ], ids=["cut_plane", "cut_line"])
-def test_other_blocks_keep_level_schedule(gen, nb):
+def test_reported_form(gen, nb):
+    # blocks that cut lines and planes run as lines too; the stored couplings
+    # are then at least the factor's
     rp, col, val = gen()
     with ph.Plan(rp, col, val, ipreflag=2, ILU_method=0, precon_thblock=nb) as P:
+        st = P.stats()
+        assert st["bj_lines"] == 1
+        assert st["bj_entries"] >= st["bj_nnz_l"] + st["bj_nnz_u"]
+    with _levels_plan(rp, col, val, ipreflag=2, ILU_method=0, precon_thblock=nb) as P:
         assert P.stats()["bj_lines"] == 0
+        assert (P.stats()["bj_levels_fwd"], P.stats()["bj_levels_bwd"]) == (st["bj_levels_fwd"], st["bj_levels_bwd"])
     with ph.Plan(rp, col, val, ipreflag=2, ILU_method=0, precon_thblock=nb, independ_nvec=2) as P:
         assert P.stats()["bj_lines"] == 0

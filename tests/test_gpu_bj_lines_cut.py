@@ -53,6 +53,7 @@ def test_apply_equals_level_scheduled(case, ilu):
         os.environ["PARCEL_HIP_BJ_LEVELS"] = levels
         try:
             with ph.Plan(rp, col, val, **kw) as P:
+                assert P.stats()["bj_lines"] == 1 - int(levels)
                 s = np.full(n, np.nan)
                 P.precon(r, s)
                 P.precon(r, s)

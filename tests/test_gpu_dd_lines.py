@@ -2,6 +2,8 @@
 against the oracle's dd PCG, bit for bit: blocks of whole lines and planes
 and blocks that cut them, one, two and four to six wavefronts per block, the
 factor's lo parts used or not.  A few iterations reach every row."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -26,12 +28,25 @@ CASES = {
 }
 
 
+def _lines(rp, col, val, ilu, nb, pp=2):
+    """Whether the plan that such a ddcg call makes runs as line wavefronts."""
+    lib, h, st = ph.load(), ctypes.c_void_p(), ph.Stats()
+    n, pt = rp.shape[0] - 1, lambda a: ctypes.c_void_p(a.ctypes.data)
+    prm = ph.default_param(ipreflag=2, ILU_method=ilu, precon_thblock=nb)
+    assert lib.parcel_hip_plan_create_dd(ctypes.byref(h), n, n, val.size, 1, pt(val), None, pt(rp), pt(col),
+                                         ctypes.byref(prm), 1, pp) == 0
+    assert lib.parcel_hip_plan_stats(h, ctypes.byref(st)) == 0
+    lib.parcel_hip_plan_destroy(h)
+    return st.as_dict()["bj_lines"]
+
+
 @pytest.mark.parametrize("ilu,pp", [(0, 2), (0, 1), (1, 2), (2, 1)])
 @pytest.mark.parametrize("case", sorted(CASES))
 def test_ddcg_bit_exact(case, ilu, pp):
     gen, nb = CASES[case]
     print("dd lines", case, ilu, pp, flush=True)
     rp, col, val = gen()
+    assert _lines(rp, col, val, ilu, nb, pp) == 1
     n = rp.shape[0] - 1
     b = ph.uniform(n, 91)
     b[:: 6] = 0.0
@@ -57,6 +72,7 @@ def test_values_beyond_the_fma_range(part, ilu):
     print("dd lines range", part, ilu, flush=True)
     nx, ny, nz = 12, 96, 6
     rp, col, val = ph.poisson3d_spd(nx, ny, nz)
+    assert _lines(rp, col, val, ilu, 3) == 1
     n = rp.shape[0] - 1
     b = ph.uniform(n, 92)
     blo = b * 2.0 ** -56
