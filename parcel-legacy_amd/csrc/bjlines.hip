@@ -174,6 +174,20 @@ struct LineArgs {
 // first, then the line neighbour, then the cell neighbour (ILU(0) keeps the
 // CRS order of the block, D-ILU walks its upper part downward); ILU(0)'s
 // backward rows hold them the other way round.
+// A wavefront's factor entries: one row of nl entries per step, lane l's entry
+// of its cell c in row c + l modulo a period of at least nx and 8 rows.  A lane
+// has at most one cell in each row of a period, and the lanes of a step share
+// their row, so the rows hold nx nl entries and no gaps (a row for each of the
+// nx + nl - 1 steps would be half empty at 64 lines of 64 cells, 8/9 at 8).  The
+// step after the period's last goes back to row 0 between groups of kLG loads
+// only: the first kLG - 1 rows stand a second time behind the period.  Few lines
+// (all their steps fit that) keep a row per step.
+inline int line_period(int nx) { return nx * ((kLG + nx - 1) / nx); }
+inline bool line_wraps(int nx, int nl, int period) { return nx + nl - 1 > period + kLG - 1; }
+inline int line_rows(int nx, int nl, int period) {
+  return line_wraps(nx, nl, period) ? period + kLG - 1 : nx + nl - 1;
+}
+
 template <bool FWD, int MODE>
 constexpr bool line_cell_first() { return !FWD && MODE == BJ_ILU0; }
 
@@ -273,8 +287,8 @@ __device__ __forceinline__ void line_sweep(const LineArgs& A, const LineBlock bk
     if (lane > 0 || wv.hand >= 0) tln = tl0 + (FWD ? nx - ls : line + nx - bk.len + 1);
     if (PL && wv.plane >= 0) tpn = tl0 + (int)(FWD ? A.nxy - ls : line + A.nxy - bk.len + 1);
   }
-  // factor entries: step t's entry of lane l at (t - tw) nl + l
-  const long ents = wv.nl > 0 ? (long)(nx + wv.nl - 1) * wv.nl : 0;
+  // the factor entries (line_period)
+  const long ents = wv.back ? (long)(wv.back / 16 + (kLG - 1) * wv.nl) : wv.nl > 0 ? (long)(nx + wv.nl - 1) * wv.nl : 0;
   typename N::Mat mc, me;
   mc.a = make_rsrc(A.c[dir][0] + 2 * wv.ebase, ents * 16);
   me.a = make_rsrc(A.e[dir][0] + NE * wv.ebase, ents * 8 * NE);
@@ -283,7 +297,11 @@ __device__ __forceinline__ void line_sweep(const LineArgs& A, const LineBlock bk
     me.b = make_rsrc(A.e[dir][1] + NE * wv.ebase, ents * 8 * NE);
   }
   const int estep = wv.nl * 16;
-  int eo = -wv.tw * estep + lane * 16;  // of the next step to load
+  int eo = wv.first + lane * 16;  // of the next load
+  // between groups of loads: a row from the period on goes back by it (one
+  // before it would become a large unsigned number; lanes without a line may go
+  // anywhere)
+  auto wrap = [&]() { eo = (int)min((unsigned)eo, (unsigned)eo - (unsigned)wv.back); };
   // An absent coupling has coefficient +0 and neighbour value kZero, whose
   // product term is -0 in the row's fma (fma(-(+0), +0, z) forward and in
   // ILU(0)'s backward rows, fma(-0, +0, z) in D-ILU's), and z + (-0) == z for
@@ -453,6 +471,7 @@ __device__ __forceinline__ void line_sweep(const LineArgs& A, const LineBlock bk
       load(u + NR, R[(p * kLG + u) % NR]);
       out.store(ov[u], chunk_off(ri - sg * 4 * 64, ci - 4 * 64, u));
     }
+    wrap();
     if (MULTI) lds_barrier();
     else wave_lds_sync();
     stage_fill(pc, sa);
@@ -480,7 +499,10 @@ __device__ __forceinline__ void line_sweep(const LineArgs& A, const LineBlock bk
   ri += sg * 64;
   ci += 64;
 #pragma unroll
-  for (int u = 0; u < NR; ++u) load(u, R[u]);
+  for (int u = 0; u < NR; ++u) {
+    load(u, R[u]);
+    if (u + 1 == NR || (u + 1) % kLG == 0) wrap();
+  }
   // the first two groups run outside the loop, so that the loop is entered
   // with the memory operations of two groups in flight on both of its paths
   // (the compiler's wait counts then match the steady state)
@@ -619,7 +641,7 @@ bool line_setup_at(Plan& P, const std::vector<BlockSweep>& F, const std::vector<
                    const std::vector<int>& blo, const std::vector<int>& bhi, int parts, long nx, long ny_plane,
                    long nxy) {
   LineBJ& G = P.M.line;
-  const int n = P.hA.n, nblk = (int)F.size(), X = (int)nx;
+  const int n = P.hA.n, nblk = (int)F.size(), X = (int)nx, period = line_period(X);
   const bool ilu0 = P.M.mode == BJ_ILU0;
   std::vector<Pieces> pc(nblk);
   int W = 1;
@@ -635,7 +657,7 @@ bool line_setup_at(Plan& P, const std::vector<BlockSweep>& F, const std::vector<
   if (line_lds_bytes(W, parts) > kLdsMax) return false;
   std::vector<LineBlock> blk(nblk);
   std::vector<LineWave> wv[2];
-  for (auto& v : wv) v.assign((size_t)nblk * W, LineWave{0, 0, 0, -1, -1, 0, 0});
+  for (auto& v : wv) v.assign((size_t)nblk * W, LineWave{0, 0, 0, -1, -1, 0, 0, 0});
   long ents = 0;
   for (int b = 0; b < nblk; ++b) {
     const Pieces& p = pc[b];
@@ -656,8 +678,13 @@ bool line_setup_at(Plan& P, const std::vector<BlockSweep>& F, const std::vector<
           // relative to lo: within (-2^31, 2^31) since a block spans less
           const long row0 = dir == 0 ? (p.first[kn] + 64L * jw) * nx : (p.first[kn] + p.ny[kn] - 64L * jw) * nx - 1;
           v.row0 = (int)(row0 - blo[b]);
-          if ((nx + v.nl - 1) * v.nl * 16 >= (1L << 30)) return false;
-          e += (nx + v.nl - 1) * v.nl;
+          const long we = (long)line_rows(X, v.nl, period) * v.nl;
+          if (we * 16 >= (1L << 30)) return false;
+          // step tw in row 0 (of some repetition of the period)
+          const bool wraps = line_wraps(X, v.nl, period);
+          v.back = wraps ? period * v.nl * 16 : 0;
+          v.first = (wraps ? (period - v.tw % period) % period : -v.tw) * v.nl * 16;
+          e += we;
           nsteps = std::max(nsteps, v.tw + v.nl - 1 + X);
         }
       ng[dir] = std::max(2, (nsteps - 1) / kLG + 3);
@@ -665,6 +692,12 @@ bool line_setup_at(Plan& P, const std::vector<BlockSweep>& F, const std::vector<
     }
     blk[b] = LineBlock{blo[b], bhi[b] - blo[b], ng[0], ng[1]};
   }
+  // Entries per row: 1.1 for whole lines of 64 cells, 1.9 at eight, 7.5 at two; a
+  // block that couples planes also holds the lines of the planes it cuts.  Beyond
+  // eight (64 bytes each in FP64, twice that in double-double) the tables would
+  // dwarf the matrix and the level form is kept; small systems (up to 64 MB
+  // more) are let through.
+  if (ents > 8L * n + (1L << 20)) return false;
   const int ne[2] = {(pl ? 1 : 0) + (ilu0 ? 0 : 1), (pl ? 1 : 0) + 1};
   const size_t pe = (size_t)std::max(parts, 1);
   std::vector<double> c[2][2], ev[2][2];
@@ -708,7 +741,10 @@ bool line_setup_at(Plan& P, const std::vector<BlockSweep>& F, const std::vector<
         const int jp = fwd ? j : p.ny[k] - 1 - j, ip = fwd ? x : X - 1 - x, kq = fwd ? k : p.np - 1 - k;
         const LineWave& v = wv[dir][(size_t)b * W + kq * p.wp + jp / 64];
         const int l = jp % 64;
-        const size_t e = (size_t)(v.ebase + (long)(ip + l) * v.nl + l);
+        const bool wraps = line_wraps(X, v.nl, period);
+        const int row = wraps ? (ip + l) % period : ip + l;
+        const size_t e = (size_t)(v.ebase + (long)row * v.nl + l);
+        const size_t again = wraps && row < kLG - 1 ? (size_t)period * v.nl : 0;  // its second place
         for (size_t q = 0; q < pe; ++q) {
           const std::vector<double>& sv = q ? S.val_lo : S.val;
           double vc = 0.0, vl = 0.0, vp = 0.0;
@@ -718,14 +754,17 @@ bool line_setup_at(Plan& P, const std::vector<BlockSweep>& F, const std::vector<
             (hc && dp == cn ? vc : hl && dp == ln ? vl : vp) = q && !lo_on ? 0.0 : sv[r];
           }
           if (bad) break;
-          c[dir][q][2 * e] = cell_first ? vc : vl;
-          c[dir][q][2 * e + 1] = cell_first ? vl : vc;
+          auto put = [&](size_t at) {
+            c[dir][q][2 * at] = cell_first ? vc : vl;
+            c[dir][q][2 * at + 1] = cell_first ? vl : vc;
+            double* t = ev[dir][q].data() + (size_t)ne[dir] * at;
+            if (pl) *t++ = vp;
+            if (ne[dir] > (pl ? 1 : 0)) *t = q ? (lo_on ? S.diag_lo[i] : 0.0) : S.diag[i];
+          };
+          put(e);
+          if (again) put(e + again);
           if (pe == 2 && q == 0 && !(dd_fma_range(vc) && dd_fma_range(vl) && dd_fma_range(vp) && dd_fma_range(S.diag[i])))
             wide = 1;
-          const double dg = q ? (lo_on ? S.diag_lo[i] : 0.0) : S.diag[i];
-          double* t = ev[dir][q].data() + (size_t)ne[dir] * e;
-          if (pl) *t++ = vp;
-          if (ne[dir] > (pl ? 1 : 0)) *t = dg;
         }
         if (bad) break;
       }
@@ -747,7 +786,6 @@ bool line_setup_at(Plan& P, const std::vector<BlockSweep>& F, const std::vector<
   G.entries = (pl ? 3 : 2) * ents;
   G.wide = wide != 0;
   G.on = true;
-  (void)n;
   return true;
 }
 

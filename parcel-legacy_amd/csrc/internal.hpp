@@ -198,7 +198,7 @@ struct LscanBJ {
 // cell of its line, the same cell of the neighbouring line and of the
 // neighbouring plane (bjlines.hip).  Per sweep and wavefront the couplings
 // and scales lie in anti-diagonal order of the wavefront's lines, so the rows
-// of one step are contiguous.
+// of one step are contiguous (bjlines.hip: line_period).
 struct LineBlock {
   int lo, len;   // the block's rows [lo, lo + len)
   int ngf, ngb;  // groups of steps of the forward / backward sweep (at least 2)
@@ -211,7 +211,8 @@ struct LineWave {
   int tw;     // the step at which lane 0 computes cell 0
   int hand;   // wavefront whose lane 63 holds the line before lane 0's (-1: none)
   int plane;  // wavefront holding the same lines of the plane before (-1: none)
-  int pad;
+  int first;  // byte offset of the first step's row of entries
+  int back;   // bytes of a period of rows (0: a row per step)
   long ebase; // first factor entry
 };
 struct LineBJ {

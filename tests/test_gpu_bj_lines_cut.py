@@ -3,7 +3,8 @@ grid lines and planes (bjlines.hip): bit for bit the level-scheduled kernel's
 result (PARCEL_HIP_BJ_LEVELS=1), signed zeros included, and solves equal to
 the oracle's.  Sizes: blocks of a line and a bit, blocks that cross a plane's
 end without coupling planes, blocks of one to four planes, one, two and six
-to eight wavefronts, odd and very short lines."""
+to eight wavefronts, odd and very short lines (the factor entries' rows then
+wrap around many times)."""
 import os
 
 import numpy as np
@@ -24,6 +25,10 @@ CASES = {
     "p2d_64x64_b7": (lambda: ph.poisson2d(64, 64, -1.0), 7),
     "p2d_37x200_b3": (lambda: ph.poisson2d(37, 200, -1.0), 3),
     "p2d_9x500_b1": (lambda: ph.poisson2d(9, 500, -1.0), 1),
+    "p2d_2x300_b1": (lambda: ph.poisson2d(2, 300, -1.0), 1),
+    "p2d_3x201_b2": (lambda: ph.poisson2d(3, 201, -1.0), 2),
+    "p2d_8x200_b3": (lambda: ph.poisson2d(8, 200, -1.0), 3),
+    "p3d_5x64x3_b1": (lambda: ph.poisson3d_spd(5, 64, 3), 1),
     "p3d_16_b3": (lambda: ph.poisson3d_spd(16, 16, 16), 3),
     "p3d_13x11x9_b20": (lambda: ph.poisson3d_spd(13, 11, 9), 20),
     "p3d_13x11x9_b85": (lambda: ph.poisson3d_spd(13, 11, 9), 85),
@@ -77,3 +82,22 @@ def test_pcg_bit_exact(case, ilu):
     xo, ho, no, io = orc.pcg(rp, col, val, b, ipreflag=2, ilu_method=ilu, nblocks=nb, itrmax=3000, rtol=1e-10)
     assert (niter, iret) == (no, io) and iret == 0
     assert np.array_equal(hist, ho) and np.array_equal(x, xo)
+
+
+@pytest.mark.parametrize("nx,ny,most", [(2, 1 << 18, 7.5), (4, 1 << 18, 3.75), (8, 1 << 17, 1.9), (64, 1 << 14, 1.2)])
+def test_narrow_grids_stay_small(nx, ny, most):
+    # 64 lines a wavefront: stored entries (a line and a cell coupling each) per row
+    print("bj lines narrow", nx, ny, flush=True)
+    rp, col, val = ph.poisson2d(nx, ny, -1.0)
+    n = rp.shape[0] - 1
+    with ph.Plan(rp, col, val, ipreflag=2, ILU_method=0, precon_thblock=ny // 64) as P:
+        st = P.stats()
+    assert st["bj_lines"] == 1 and st["bj_entries"] <= 2 * 2 * most * n
+
+
+def test_padding_beyond_the_bound_keeps_levels():
+    # blocks of 1.05 planes hold the lines of two or three, of two cells each
+    print("bj lines bound", flush=True)
+    rp, col, val = ph.poisson3d_spd(2, 64, 1 << 13)
+    with ph.Plan(rp, col, val, ipreflag=2, ILU_method=0, precon_thblock=int((1 << 13) / 1.05)) as P:
+        assert P.stats()["bj_lines"] == 0

@@ -20,6 +20,8 @@ def _init():
 
 CASES = {
     "p2d_40x70_b3": (lambda: ph.poisson2d(40, 70, -1.0), 3),
+    "p2d_3x201_b2": (lambda: ph.poisson2d(3, 201, -1.0), 2),
+    "p2d_8x150_b1": (lambda: ph.poisson2d(8, 150, -1.0), 1),
     "p3d_20_b20": (lambda: ph.poisson3d_spd(20, 20, 20), 20),
     "p3d_13x11x9_b20": (lambda: ph.poisson3d_spd(13, 11, 9), 20),
     "p3d_20_b7": (lambda: ph.poisson3d_spd(20, 20, 20), 7),
