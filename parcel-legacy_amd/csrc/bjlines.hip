@@ -637,9 +637,64 @@ Pieces pieces_of(int lo, int hi, long nx, long ny_plane, long nxy) {
   return p;
 }
 
+// Whether a dependency of the sweeps lies more than three levels back, beyond
+// the LDS ring of the level-scheduled kernels.
+bool beyond_ring(const std::vector<BlockSweep>& F, const std::vector<BlockSweep>& B) {
+  int far = 0;
+#pragma omp parallel for schedule(dynamic) reduction(| : far)
+  for (size_t b = 0; b < F.size(); ++b)
+    for (const BlockSweep* S : {&F[b], &B[b]}) {
+      std::vector<int> lev(S->diag.size());
+      for (size_t l = 0; l + 1 < S->lev_start.size(); ++l)
+        for (int t = S->lev_start[l]; t < S->lev_start[l + 1]; ++t) lev[S->order[t]] = (int)l;
+      for (size_t i = 0; i < lev.size() && !far; ++i)
+        for (int q = S->ptr[i]; q < S->ptr[i + 1]; ++q)
+          if (lev[i] - lev[S->dep[q]] > 3) far = 1;
+    }
+  return far != 0;
+}
+
+// Whether line wavefronts are the faster form: `waves` wavefronts a block and
+// `groups` groups of steps in both sweeps, against the levels of both sweeps.
+// Lines cost groups, however few lanes a group has at work, so many small
+// planes in a block, or many wavefronts of two to eight cells a line, are the
+// levels' (2048 blocks of eight 8 x 8 planes: 91 us level by level, 452 as
+// lines; 1024 blocks of four 16 x 16 planes 70 and 116; 512 blocks of 512 lines
+// of four cells 368 and 554), all else the lines' (up to 7 times faster).  The
+// estimates, in us, take the longer of one block's chain, the work of all
+// blocks on the device, and memory; fitted to 255 FP64 and 105 double-double
+// block shapes of 2^12 to 2^22 rows, within 15 % (rms).  On these the form taken
+// is the faster one but for six, where it costs 3 to 12 % (FP64) and 20 and 34 %
+// (double-double).
+bool line_pays(int device, const std::vector<BlockSweep>& F, const std::vector<BlockSweep>& B, int n, int waves,
+               int groups, bool planes, int parts) {
+  int cu = 0;
+  if (hipDeviceGetAttribute(&cu, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || cu < 1) return true;
+  const double nblk = (double)F.size(), dd = parts == 2;
+  int levels = 0, width = 1;
+  for (size_t b = 0; b < F.size(); ++b) {
+    int l = 0;
+    for (const BlockSweep* S : {&F[b], &B[b]}) {
+      l += std::max(0, (int)S->lev_start.size() - 1);
+      for (size_t k = 0; k + 1 < S->lev_start.size(); ++k)
+        width = std::max(width, S->lev_start[k + 1] - S->lev_start[k]);
+    }
+    levels = std::max(levels, l);
+  }
+  const double chain = groups * (planes ? 1.15 : 0.86) * (waves > 4 ? (dd ? 1.5 : 2.0) : 1.0);
+  const double work = nblk * waves * groups / (4.0 * cu) * (planes ? 1.47 : 0.95);
+  const double line = std::max({chain, work, n * 1.3e-5}) * (dd ? 3.0 : 1.0) + 2.0;
+  auto level = [&](double slow) {
+    return std::max({levels * (planes ? 0.37 : 0.29), nblk * levels / cu * (planes ? 0.24 : 0.19), n * 5.5e-5}) *
+               (slow * (dd ? 2.5 : 1.0)) + 4.0;
+  };
+  const double wide = width <= 256 ? 1.0 : width <= 512 ? 1.9 : 6.0;  // wavefronts a level needs; past 512 unpipelined
+  return line <= level(wide) || (line <= level(2.0 * wide) && beyond_ring(F, B));
+}
+
 bool line_setup_at(Plan& P, const std::vector<BlockSweep>& F, const std::vector<BlockSweep>& B,
-                   const std::vector<int>& blo, const std::vector<int>& bhi, int parts, long nx, long ny_plane,
-                   long nxy) {
+                   const std::vector<int>& blo, const std::vector<int>& bhi, int parts, bool forced, long nx,
+                   long ny_plane, long nxy) {
   LineBJ& G = P.M.line;
   const int n = P.hA.n, nblk = (int)F.size(), X = (int)nx, period = line_period(X);
   const bool ilu0 = P.M.mode == BJ_ILU0;
@@ -698,6 +753,11 @@ bool line_setup_at(Plan& P, const std::vector<BlockSweep>& F, const std::vector<
   // dwarf the matrix and the level form is kept; small systems (up to 64 MB
   // more) are let through.
   if (ents > 8L * n + (1L << 20)) return false;
+  if (!forced) {
+    int groups = 0;
+    for (const LineBlock& k : blk) groups = std::max(groups, k.ngf + k.ngb);
+    if (!line_pays(P.device, F, B, n, W, groups, pl, parts)) return false;
+  }
   const int ne[2] = {(pl ? 1 : 0) + (ilu0 ? 0 : 1), (pl ? 1 : 0) + 1};
   const size_t pe = (size_t)std::max(parts, 1);
   std::vector<double> c[2][2], ev[2][2];
@@ -821,12 +881,16 @@ void launch_lines(K kern, int nblocks, int waves, size_t shm, hipStream_t st, Ar
 // are 1, nx and (blocks longer than a plane) nxy; where no block couples
 // planes the matrix's first row gives the lines per plane, and if the rows do
 // not fit that, every line but the first is tried with a line neighbour.
-// PARCEL_HIP_BJ_LEVELS=1 in the environment keeps the level-scheduled apply.
+// PARCEL_HIP_BJ_LEVELS=1 in the environment keeps the level-scheduled apply, =0
+// takes the lines also where line_pays would not.
 bool line_setup(Plan& P, const std::vector<BlockSweep>& F, const std::vector<BlockSweep>& B,
                 const std::vector<int>& blo, const std::vector<int>& bhi, int parts) {
   P.M.line = LineBJ();
-  if (const char* e = std::getenv("PARCEL_HIP_BJ_LEVELS"))
+  bool forced = false;
+  if (const char* e = std::getenv("PARCEL_HIP_BJ_LEVELS")) {
     if (e[0] && e[0] != '0') return false;
+    forced = e[0] == '0';
+  }
   const int n = P.hA.n, nblk = (int)F.size();
   for (int b = 0; b + 1 < nblk; ++b)
     if (bhi[b] != blo[b + 1]) return false;
@@ -842,15 +906,15 @@ bool line_setup(Plan& P, const std::vector<BlockSweep>& F, const std::vector<Blo
       }
   if (o1 && o2 && o2 < o1) std::swap(o1, o2);
   if (o1 < 2 || o1 >= (1L << 24) || (o2 && o2 % o1)) return false;
-  if (o2) return line_setup_at(P, F, B, blo, bhi, parts, o1, o2 / o1, o2);
+  if (o2) return line_setup_at(P, F, B, blo, bhi, parts, forced, o1, o2 / o1, o2);
   // blocks without plane couplings: the other offset of the matrix's first
   // row, which has every forward neighbour of a grid
   const HostCSR& A = P.hA;
   long m2 = 0;
   for (int e = A.rowptr[0]; e < A.rowptr[1]; ++e) m2 = std::max(m2, (long)A.col[e]);
   const long all = (n + o1 - 1) / o1;
-  if (m2 > o1 && m2 % o1 == 0 && line_setup_at(P, F, B, blo, bhi, parts, o1, m2 / o1, 0)) return true;
-  return line_setup_at(P, F, B, blo, bhi, parts, o1, all, 0);
+  if (m2 > o1 && m2 % o1 == 0 && line_setup_at(P, F, B, blo, bhi, parts, forced, o1, m2 / o1, 0)) return true;
+  return line_setup_at(P, F, B, blo, bhi, parts, forced, o1, all, 0);
 }
 
 void line_apply(Plan& P, const double* r, double* s, const CGFuse* fuse, const int* skip) {

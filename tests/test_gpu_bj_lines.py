@@ -54,8 +54,8 @@ SYM = ("p3d_16_b16", "p3d_48x100x6_b6", "p2d_100x300_b2", "p2d_40x512_b1", "p3d_
        "p3d_16x100x4_b2_planes2", "p3d_10x30x16_b4_planes4")
 
 
-def _levels_plan(rp, col, val, **kw):
-    os.environ["PARCEL_HIP_BJ_LEVELS"] = "1"
+def _levels_plan(rp, col, val, levels="1", **kw):
+    os.environ["PARCEL_HIP_BJ_LEVELS"] = levels
     try:
         return ph.Plan(rp, col, val, **kw)
     finally:
@@ -134,7 +134,7 @@ def test_reported_form(gen, nb):
     # blocks that cut lines and planes run as lines too; the stored couplings
     # are then at least the factor's
     rp, col, val = gen()
-    with ph.Plan(rp, col, val, ipreflag=2, ILU_method=0, precon_thblock=nb) as P:
+    with _levels_plan(rp, col, val, levels="0", ipreflag=2, ILU_method=0, precon_thblock=nb) as P:
         st = P.stats()
         assert st["bj_lines"] == 1
         assert st["bj_entries"] >= st["bj_nnz_l"] + st["bj_nnz_u"]
@@ -143,3 +143,23 @@ def test_reported_form(gen, nb):
         assert (P.stats()["bj_levels_fwd"], P.stats()["bj_levels_bwd"]) == (st["bj_levels_fwd"], st["bj_levels_bwd"])
     with ph.Plan(rp, col, val, ipreflag=2, ILU_method=0, precon_thblock=nb, independ_nvec=2) as P:
         assert P.stats()["bj_lines"] == 0
+
+
+@pytest.mark.parametrize("grid,nb,lines", [
+    ((8, 8, 512), 64, 0),        # eight planes of eight lines: 8 of 64 lanes in eight wavefronts
+    ((8, 8, 512), 128, 0),       # four planes
+    ((16, 16, 4096), 1024, 0),   # four planes of 16 lines
+    ((16, 16, 4096), 4096, 1),   # one
+    ((32, 32, 64), 16, 1),       # four planes of 32 lines
+    ((75, 61, 43), 256, 1),      # ten lines and a bit
+    ((64, 64, 20), 8, 1),        # two and a half planes
+    ((4, 1 << 18), 512, 0),      # 512 lines of four cells
+    ((4, 1 << 18), 4096, 1),     # 64 of them
+    ((300, 300), 2, 1),
+])
+def test_form_by_the_rule(grid, nb, lines):
+    # the faster form of both, as measured
+    say("bj lines rule", grid, nb)
+    gen = ph.poisson3d_spd(*grid) if len(grid) == 3 else ph.poisson2d(*grid, -1.0)
+    with ph.Plan(*gen, ipreflag=2, ILU_method=0, precon_thblock=nb) as P:
+        assert P.stats()["bj_lines"] == lines

@@ -18,7 +18,11 @@ pytestmark = pytest.mark.gpu
 
 @pytest.fixture(scope="module", autouse=True)
 def _init():
+    # PARCEL_HIP_BJ_LEVELS=0: line wavefronts also where the levels are faster
     ph.init(0)
+    os.environ["PARCEL_HIP_BJ_LEVELS"] = "0"
+    yield
+    del os.environ["PARCEL_HIP_BJ_LEVELS"]
 
 
 CASES = {
@@ -64,7 +68,7 @@ def test_apply_equals_level_scheduled(case, ilu):
                 P.precon(r, s)
                 out.append(s)
         finally:
-            del os.environ["PARCEL_HIP_BJ_LEVELS"]
+            os.environ["PARCEL_HIP_BJ_LEVELS"] = "0"
     assert np.array_equal(out[0].view(np.uint64), out[1].view(np.uint64))
 
 

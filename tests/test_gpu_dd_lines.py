@@ -3,6 +3,7 @@ against the oracle's dd PCG, bit for bit: blocks of whole lines and planes
 and blocks that cut them, one, two and four to six wavefronts per block, the
 factor's lo parts used or not.  A few iterations reach every row."""
 import ctypes
+import os
 
 import numpy as np
 import pytest
@@ -15,7 +16,11 @@ pytestmark = pytest.mark.gpu
 
 @pytest.fixture(scope="module", autouse=True)
 def _init():
+    # PARCEL_HIP_BJ_LEVELS=0: line wavefronts also where the levels are faster
     ph.init(0)
+    os.environ["PARCEL_HIP_BJ_LEVELS"] = "0"
+    yield
+    del os.environ["PARCEL_HIP_BJ_LEVELS"]
 
 
 CASES = {
