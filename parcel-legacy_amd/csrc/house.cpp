@@ -15,6 +15,7 @@
 
 namespace parcel {
 
+#if defined(__x86_64__)
 namespace {
 
 // Rows of S: element (j, k) at S[j * N + k].
@@ -75,5 +76,8 @@ bool house_r_rows(int m, int n, double* S, double* R) {
     default: return false;
   }
 }
+#else  // the caller's column loops
+bool house_r_rows(int, int, double*, double*) { return false; }
+#endif
 
 }  // namespace parcel
