@@ -640,6 +640,9 @@ void batch_cg_loop(Batch& B, const BVecs<T>& V, TZ* z, T* x, const T* b, int itr
   PARCEL_HIP_CHECK(hipGetLastError());
   B.hstate.ensure((size_t)nsys);
   CGState* h = B.hstate.p;
+  // fixed chunks, not ChunkRule's: the loop ends with the slowest of the systems,
+  // which a look at one residual does not foretell, and an iteration of many
+  // systems is long beside the launches after the end
   int enq = 0, chunk = 8;
   bool all_done = false;
   while (enq < itrmax + 1) {

@@ -24,21 +24,27 @@
 //
 // What bounds it: with few blocks (64 on 256 CUs) the sweep is one dependent
 // chain of steps and a lone wavefront per SIMD issues an instruction per four
-// cycles at best, so the instructions of a step are the time: the factor
+// cycles at best, so the instructions of a step are the time (64 blocks of two
+// 128 x 128 planes: a wavefront issues in 46 % of its cycles): the factor
 // operands lie in anti-diagonal order (lane l's entry of a step is contiguous),
 // addresses advance by constants, every access goes through a buffer
 // descriptor whose bounds check drops the lanes off the block (no selects of
 // addresses, no sink stores, no branches), all ring slots are immediate
 // offsets, and both streams are loaded two groups ahead.  With one block per
-// CU (256 planes of 256 x 256) HBM bounds it.
+// CU (256 planes of 256 x 256) HBM bounds it: 1.3 GB of traffic at 4.65 TB/s,
+// near a copy's 4.75.  With six wavefronts a block on four SIMDs (80 blocks of
+// two 160 x 160 planes) a wavefront issues in 22 % of its cycles and waits to
+// issue in 55 %, at 2.0 TB/s: neither HBM nor the instruction count, but SIMDs
+// that two wavefronts share and a barrier of all six every eight steps.
 // Measured, one apply, against the kernels before (a line form for whole lines
 // and planes with addresses selected per lane; level-scheduled sweeps for the
 // others): 64 blocks of two 128 x 128 planes ILU(0) 157 -> 92 us; 256 planes of
-// 256 x 256 with the fused update 340 -> 313 us in the solve; 80 blocks of two
+// 256 x 256 with the fused update 388 -> 353 us in the solve; 80 blocks of two
 // 160 x 160 planes D-ILU 813 -> 199 us; 256 blocks of 10 1/4 lines of 75 cells
 // D-ILU 136 -> 23 us.  Double-double, 32 blocks of three 96 x 96 planes ILU(0)
 // (level-scheduled before): 675 -> 284 us (350 with Dekker's products), bound
-// by FP64 issue (six wavefronts on four SIMDs).
+// by FP64 issue (a wavefront issues in 44 % of its cycles, and two of the four
+// SIMDs hold two).
 #include <algorithm>
 #include <cstdlib>
 #include <type_traits>

@@ -320,8 +320,10 @@ __global__ void __launch_bounds__(kNT) k_cg_spmv(int n, int it, int itrmax, doub
   const long ntiles = ((long)n + kNT - 1) / kNT;
   // stencil form: the first trip's operands, in flight while the state is read
   // and the partials are reduced (they depend on neither): a small system's
-  // launch waits for one memory round trip less (256^2: 5.7 -> 5.25 us; FP32
-  // 256^3: 153 -> 144 us, FP64 318 -> 310 us)
+  // launch waits for one memory round trip less (with k_cg_update_pj's, 400
+  // iterations of point-Jacobi CG: 200^2 4.68 -> 4.34 ms, 1000^2 13.8 -> 12.6,
+  // 2048 x 1024 21.3 -> 19.8; a launch on 256^3 in FP32 169 -> 158 us, in FP64
+  // 353 before and 358 now)
   constexpr bool kPre = IsSt7<MT>::value && LB == 1;
   constexpr int U = kSt7U;
   const long stride = (long)nb * kNT;
@@ -447,7 +449,7 @@ __global__ void __launch_bounds__(kNT) k_cg_update_pj(int n, int it, T* __restri
   const int nb = gridDim.x;
   const long ntiles = ((long)n + kNT - 1) / kNT;
   // the first tile's operands, in flight while the state is read and the
-  // partials are reduced (256^2: 3.6 -> 3.36 us)
+  // partials are reduced (256^2: 3.9 -> 3.6 us)
   long i = (long)tile_owner() * kNT + threadIdx.x;
   T r0 = 0, q0 = 0, d0 = 1;
   auto load = [&]() {
