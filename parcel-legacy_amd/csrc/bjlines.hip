@@ -262,6 +262,10 @@ struct FmaRange {
   __device__ __forceinline__ bool outside() const { return lo < (unsigned)(kFmaLo - 1) || hi >= kFmaHi - 1; }
 };
 
+// Of a sweep's groups, those that have steps (two at least: line_sweep peels
+// them); the others bring the last chunks out of the ring.
+__host__ __device__ __forceinline__ int line_sweep_groups(int ng) { return ng - 2 > 2 ? ng - 2 : 2; }
+
 // One sweep of a block.  NR: steps the factor operands are loaded ahead.
 // alphaf: the fused update's alpha, asked for once the first loads are out.
 template <bool FWD, int MODE, bool FUSED, bool PL, bool MULTI, int NV, int NR, bool FMA = false, class AF>
@@ -514,9 +518,23 @@ __device__ __forceinline__ void line_sweep(const LineArgs& A, const LineBlock bk
   // (the compiler's wait counts then match the steady state)
   group(P0{});
   group(P1{});
-  for (int g = 2; g < ng; g += 2) {
+  const int nf = line_sweep_groups(ng);
+  for (int g = 2; g < nf; g += 2) {
     group(P0{});
-    if (g + 1 < ng) group(P1{});
+    if (g + 1 < nf) group(P1{});
+  }
+  // every step is done: the last chunks out of the ring (with whole groups here,
+  // 65536 blocks of 2 x 8 cells took 570 us an apply, 433 now; 256 of ten lines of
+  // 75 cells 23.4 and 21.7)
+  for (int g = nf; g < ng; ++g) {
+    wave_lds_sync();
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+      out.store(N::get(stg[8 * k * kLL + sa]), chunk_off(ri - sg * 4 * 64, ci - 4 * 64, k));
+    ri += sg * 64;
+    ci += 64;
+    sa = sb;
+    sb = next_slot(sb);
   }
 }
 
@@ -664,14 +682,14 @@ bool beyond_ring(const std::vector<BlockSweep>& F, const std::vector<BlockSweep>
 // `groups` groups of steps in both sweeps, against the levels of both sweeps.
 // Lines cost groups, however few lanes a group has at work, so many small
 // planes in a block, or many wavefronts of two to eight cells a line, are the
-// levels' (2048 blocks of eight 8 x 8 planes: 91 us level by level, 452 as
-// lines; 1024 blocks of four 16 x 16 planes 70 and 116; 512 blocks of 512 lines
-// of four cells 368 and 554), all else the lines' (up to 7 times faster).  The
-// estimates, in us, take the longer of one block's chain, the work of all
-// blocks on the device, and memory; fitted to 255 FP64 and 105 double-double
-// block shapes of 2^12 to 2^22 rows, within 15 % (rms).  On these the form taken
-// is the faster one but for six, where it costs 3 to 12 % (FP64) and 20 and 34 %
-// (double-double).
+// levels' (2048 blocks of eight 8 x 8 planes: 91 us level by level, 402 as
+// lines; 1024 blocks of four 16 x 16 planes 70 and 103; 512 blocks of 512 lines
+// of four cells 369 and 542), all else the lines' (up to 7 times faster).  The
+// estimates, in us (less what both forms spend alike), take the longer of one
+// block's chain, the work of all blocks on the device, and memory; fitted to 264
+// FP64 and 105 double-double block shapes of 2^12 to 2^22 rows, within 16 % (rms).
+// On these the form taken is the faster one, but for two double-double shapes
+// where it costs 13 and 17 %.
 bool line_pays(int device, const std::vector<BlockSweep>& F, const std::vector<BlockSweep>& B, int n, int waves,
                int groups, bool planes, int parts) {
   int cu = 0;
@@ -688,11 +706,11 @@ bool line_pays(int device, const std::vector<BlockSweep>& F, const std::vector<B
     levels = std::max(levels, l);
   }
   const double chain = groups * (planes ? 1.15 : 0.86) * (waves > 4 ? (dd ? 1.5 : 2.0) : 1.0);
-  const double work = nblk * waves * groups / (4.0 * cu) * (planes ? 1.47 : 0.95);
-  const double line = std::max({chain, work, n * 1.3e-5}) * (dd ? 3.0 : 1.0) + 2.0;
+  const double work = nblk * waves * groups / (4.0 * cu) * (planes ? 1.55 : 0.95);
+  const double line = std::max({chain, work, n * 1.3e-5}) * (dd ? 3.0 : 1.0);
   auto level = [&](double slow) {
     return std::max({levels * (planes ? 0.37 : 0.29), nblk * levels / cu * (planes ? 0.24 : 0.19), n * 5.5e-5}) *
-               (slow * (dd ? 2.5 : 1.0)) + 4.0;
+               (slow * (dd ? 2.5 : 1.0));
   };
   const double wide = width <= 256 ? 1.0 : width <= 512 ? 1.9 : 6.0;  // wavefronts a level needs; past 512 unpipelined
   return line <= level(wide) || (line <= level(2.0 * wide) && beyond_ring(F, B));
@@ -761,7 +779,7 @@ bool line_setup_at(Plan& P, const std::vector<BlockSweep>& F, const std::vector<
   if (ents > 8L * n + (1L << 20)) return false;
   if (!forced) {
     int groups = 0;
-    for (const LineBlock& k : blk) groups = std::max(groups, k.ngf + k.ngb);
+    for (const LineBlock& k : blk) groups = std::max(groups, line_sweep_groups(k.ngf) + line_sweep_groups(k.ngb));
     if (!line_pays(P.device, F, B, n, W, groups, pl, parts)) return false;
   }
   const int ne[2] = {(pl ? 1 : 0) + (ilu0 ? 0 : 1), (pl ? 1 : 0) + 1};
