@@ -31,18 +31,18 @@
 // descriptor whose bounds check drops the lanes off the block (no selects of
 // addresses, no sink stores, no branches), all ring slots are immediate
 // offsets, and both streams are loaded two groups ahead.  With one block per
-// CU (256 planes of 256 x 256) HBM bounds it: 1.3 GB of traffic at 4.65 TB/s,
+// CU (256 planes of 256 x 256) HBM bounds it: 1.3 GB of traffic at 4.70 TB/s,
 // near a copy's 4.75.  With six wavefronts a block on four SIMDs (80 blocks of
 // two 160 x 160 planes) a wavefront issues in 22 % of its cycles and waits to
-// issue in 55 %, at 2.0 TB/s: neither HBM nor the instruction count, but SIMDs
+// issue in 55 %, at 2.1 TB/s: neither HBM nor the instruction count, but SIMDs
 // that two wavefronts share and a barrier of all six every eight steps.
 // Measured, one apply, against the kernels before (a line form for whole lines
 // and planes with addresses selected per lane; level-scheduled sweeps for the
-// others): 64 blocks of two 128 x 128 planes ILU(0) 157 -> 92 us; 256 planes of
-// 256 x 256 with the fused update 388 -> 353 us in the solve; 80 blocks of two
-// 160 x 160 planes D-ILU 813 -> 199 us; 256 blocks of 10 1/4 lines of 75 cells
-// D-ILU 136 -> 23 us.  Double-double, 32 blocks of three 96 x 96 planes ILU(0)
-// (level-scheduled before): 675 -> 284 us (350 with Dekker's products), bound
+// others): 64 blocks of two 128 x 128 planes ILU(0) 157 -> 89 us; 256 planes of
+// 256 x 256 with the fused update 388 -> 351 us in the solve; 80 blocks of two
+// 160 x 160 planes D-ILU 813 -> 190 us; 256 blocks of 10 1/4 lines of 75 cells
+// D-ILU 136 -> 22 us.  Double-double, 32 blocks of three 96 x 96 planes ILU(0)
+// (level-scheduled before): 675 -> 268 us (350 with Dekker's products), bound
 // by FP64 issue (a wavefront issues in 44 % of its cycles, and two of the four
 // SIMDs hold two).
 #include <algorithm>
@@ -605,7 +605,7 @@ __global__ void __launch_bounds__(NTH) k_bj_lines_dd(LineArgs A, const double* r
   const Vec vs = line_vec<2>(sh, sl, bk), vr = line_vec<2>(rh, rl, bk);
   dd16* lds = reinterpret_cast<dd16*>(lds_lines);
   // lds_lines asks for 16-byte alignment because of this: 8 bytes off, the
-  // rings' 128-bit accesses took the apply from 284 to 502 us
+  // rings' 128-bit accesses took the apply from 284 (then) to 502 us
   __shared__ int outside;
   if (threadIdx.x == 0) outside = 0;
   auto none = []() -> double { return 0.0; };
